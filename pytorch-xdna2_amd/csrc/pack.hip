@@ -108,49 +108,26 @@ __device__ inline int tile_piece(int pix, int q) {
 constexpr int kMaxTilePix = 256;   // pixels per workgroup (LDS 32 KiB: four workgroups per CU)
 
 // Writes the 16-byte piece q of packed row p (main copy and, for the first 78 rows of a
-// group, the halo copy at the end of the previous group), when p is in [plo, phi).
-__device__ inline void put_row_piece(uint16_t* __restrict__ dst, int64_t p, int q, uint4 v,
-                                     int chunks, int chunk, int g0, int ng, int64_t plo,
-                                     int64_t phi) {
-  if (p < plo || p >= phi) return;
+// group, the halo copy at the end of the previous group).
+__device__ inline void put_row_piece(uint16_t* __restrict__ dst, int64_t p, int q, uint4 v, int chunks, int chunk,
+                                     int groups) {
   const int64_t g = p / kGroupOutRows;
   const int r = int(p - g * kGroupOutRows);
-  if (g >= g0 && g < int64_t(g0) + ng)
-    *reinterpret_cast<uint4*>(dst + ((int64_t(g - g0) * chunks + chunk) * kGroupRows + r) * kKStep + q * 8) = v;
-  if (g > g0 && g <= int64_t(g0) + ng && r + kGroupOutRows < kGroupRows)
-    *reinterpret_cast<uint4*>(dst + ((int64_t(g - 1 - g0) * chunks + chunk) * kGroupRows + r + kGroupOutRows) *
-                                        kKStep + q * 8) = v;
+  if (g < groups) *reinterpret_cast<uint4*>(dst + ((g * chunks + chunk) * kGroupRows + r) * kKStep + q * 8) = v;
+  if (g > 0 && r + kGroupOutRows < kGroupRows)
+    *reinterpret_cast<uint4*>(dst + (((g - 1) * chunks + chunk) * kGroupRows + r + kGroupOutRows) * kKStep + q * 8) = v;
 }
 
-// kDense = false: only rows of real pixels and only the real channels are written (the
-// reference's contract: the caller zero-fills once per shape).  kDense = true: every
-// element of groups [g0, g0 + ng) is written, zeros included (border rows and columns,
-// padded channels, the rows past the last image), so a buffer needs no fill; workgroups
-// from nimg on write the rows past the last image.
-// kDil (dense only): the packed image is the H x W spread of src, whose planes are
-// ceil(H/2) x ceil(W/2): pixel (y, x) = src[y/2][x/2] at even y and x, 0 elsewhere (the
-// gradient of a stride-2 conv on the stride-1 grid).  R is even, so a workgroup's full
-// rows [y0, y0 + R) read the source rows [y0/2, y0/2 + R/2) and the LDS tile holds those.
-template <int VP, bool kDense, bool kDil = false>
+// Only rows of real pixels and only the real channels are written (the reference's
+// contract: the caller zero-fills once per shape).
+template <int VP>
 __global__ __launch_bounds__(256) void pack_rows_lds_kernel(
     const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int C, int H, int W, int S,
     int So, int Wg, int wp, int lead, int halo_zero, int chunks, int g0, int ng, int b0, int64_t plo,
-    int64_t phi, int R, int ybl, int nimg, int64_t tail0) {
+    int64_t phi, int R, int ybl) {
   extern __shared__ __attribute__((aligned(16))) uint16_t tile[];
   constexpr int kVpShift = VP == 4 ? 2 : VP == 2 ? 1 : 0;
   int bid = blockIdx.x;
-  if (kDense && bid >= nimg) {
-    // rows [tail0, phi) hold no image: zeros for every chunk
-    const int64_t n = (phi - tail0) * chunks * 8;
-    const uint4 z = make_uint4(0, 0, 0, 0);
-    for (int64_t i = int64_t(bid - nimg) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x - nimg) * 256) {
-      const int q = int(i & 7);
-      const int64_t rc = i >> 3;
-      const int chunk = int(rc % chunks);
-      put_row_piece(dst, tail0 + rc / chunks, q, z, chunks, chunk, g0, ng, plo, phi);
-    }
-    return;
-  }
   const int yb = bid % ybl;
   bid /= ybl;
   const int chunk = bid % chunks;
@@ -159,12 +136,9 @@ __global__ __launch_bounds__(256) void pack_rows_lds_kernel(
   if (cc <= 0) return;
   const int y0 = yb * R;
   const int rows = min(R, H - y0);
-  // source planes: H x W, or ceil(H/2) x ceil(W/2) spread over H x W (kDil)
-  const int Hs = kDil ? (H + 1) >> 1 : H, Ws = kDil ? (W + 1) >> 1 : W;
-  const int ys0 = kDil ? y0 >> 1 : y0;
-  const int npix = (kDil ? min((rows + 1) >> 1, Hs - ys0) : rows) * Ws;
-  const int64_t plane = int64_t(Hs) * Ws;
-  const uint16_t* sbase = src + (int64_t(b) * C + chunk * kKStep) * plane + int64_t(ys0) * Ws;
+  const int npix = rows * W;
+  const int64_t plane = int64_t(H) * W;
+  const uint16_t* sbase = src + (int64_t(b) * C + chunk * kKStep) * plane + int64_t(y0) * W;
   // phase 1: NCHW rows [y0, y0 + rows) -> tile[pix][c], pix = yy * W + x.  An item is
   // VP consecutive pixels x 16 channels: 16 loads of VP pixels each (one per channel, all
   // issued before the first LDS write), then VP x two 16-byte LDS writes.
@@ -183,7 +157,7 @@ __global__ __launch_bounds__(256) void pack_rows_lds_kernel(
         uint2 t = make_uint2(0, 0);
         if (ok) t = *reinterpret_cast<const uint2*>(sp + k * plane);
         d[k][0] = t.x;
-        d[k][1] = t.y;
+        d[k][VP == 4 ? 1 : 0] = t.y;
       } else if (VP == 2) {
         d[k][0] = ok ? *reinterpret_cast<const uint32_t*>(sp + k * plane) : 0u;
       } else {
@@ -211,37 +185,6 @@ __global__ __launch_bounds__(256) void pack_rows_lds_kernel(
   __syncthreads();
 
   // phase 2: packed rows of every strip (and the halo copies into the previous group)
-  if (kDense) {
-    // grid rows y0+1 .. y0+rows (plus the top / bottom border row for the first / last
-    // tile), all wp columns, all 64 channels
-    const int gy_lo = y0 == 0 ? 0 : y0 + 1;
-    const int gy_hi = y0 + rows == H ? H + 2 : y0 + rows + 1;
-    const int grows = gy_hi - gy_lo;
-    const int nst = S * grows * wp * 8;
-    for (int t = threadIdx.x; t < nst; t += 256) {
-      const int q = t & 7;
-      const int opix = t >> 3;
-      const int s = opix / (grows * wp);
-      const int rem = opix - s * (grows * wp);
-      const int gr = rem / wp, gx = rem - gr * wp;
-      const int gy = gy_lo + gr;
-      const int j = gx - lead;
-      const int x = (S == 1 ? 0 : s * So - 1) + j;
-      const bool zero_col = halo_zero && S > 1 && (j == 0 || j == Wg - 1);
-      uint4 v = make_uint4(0, 0, 0, 0);
-      const bool real = gy >= 1 && gy <= H && j >= 0 && j < Wg && x >= 0 && x < W && !zero_col && q * 8 < cc;
-      if (kDil) {
-        // image row gy - 1 and column x even: source pixel ((gy - 1) / 2, x / 2)
-        if (real && ((gy - 1) & 1) == 0 && (x & 1) == 0)
-          v = *reinterpret_cast<const uint4*>(tile + tile_piece<kVpShift>((((gy - 1) >> 1) - ys0) * Ws + (x >> 1), q));
-      } else if (real) {
-        v = *reinterpret_cast<const uint4*>(tile + tile_piece<kVpShift>((gy - 1 - y0) * W + x, q));
-      }
-      const int64_t p = ((int64_t(b) * S + s) * (H + 2) + gy) * wp + gx;
-      put_row_piece(dst, p, q, v, chunks, chunk, g0, ng, plo, phi);
-    }
-    return;
-  }
   const int nseg = (cc + 7) >> 3;
   const int spix = rows * Wg;  // packed rows per strip
   const int nst = S * spix * nseg;
@@ -275,6 +218,154 @@ __global__ __launch_bounds__(256) void pack_rows_lds_kernel(
       } else {
         for (int c = q * 8; c < cc; ++c) d[c] = zero ? uint16_t(0) : tp[c - q * 8];
       }
+    }
+  }
+}
+
+// Four pixels of one channel: an 8-byte load at the alignment the plane offsets leave
+// (global loads take any 2-byte address on gfx950).
+struct __attribute__((packed, aligned(2))) Pix4 {
+  uint32_t lo, hi;
+};
+
+// n / d for n * d < 2^32 and d > 1, with m = 0xFFFFFFFF / d + 1: one multiply instead of
+// the ~20 instructions of a division by a run-time value.
+__device__ inline int fast_div(int n, uint32_t m) { return int(__umulhi(uint32_t(n), m)); }
+
+// The dense pack of the conv path: every element of every group is written, zeros included
+// (border rows and columns, padded channels, the rows past the last image), so a buffer
+// needs no fill; workgroups from nimg on write the rows past the last image.
+// kDil: the packed image is the H x W spread of src, whose planes are ceil(H/2) x
+// ceil(W/2): pixel (y, x) = src[y/2][x/2] at even y and x, 0 elsewhere (the gradient of a
+// stride-2 conv on the stride-1 grid).  R is even, so a workgroup's full rows
+// [y0, y0 + R) read the source rows [y0/2, y0/2 + R/2) and the LDS tile holds those.
+//
+// Large images are bound by HBM, the layers of a small network by the latency of load ->
+// LDS -> store and by index arithmetic.  So: every run takes 4-pixel loads whatever its
+// alignment (a run's last group is moved back to end with the run and rewrites pixels of
+// its neighbour with the same values; VP = 1 only where a run is shorter than 4 pixels),
+// all 16 of an item's loads are unconditional (channels past the last read it again and
+// are dropped), and the packed row of a piece is the strip's first row plus the piece's
+// index, so phase 2 divides once, by a multiplication, and keeps 32-bit offsets.  Against
+// one kernel for this and the zero-filled contract above, with run-time divisions and
+// element loads for odd planes (us in a graph, MI355X): 7x48x29x43 7.95 -> 3.94,
+// 40x128x9x9 4.76 -> 3.28, 16x128x36x36 6.09 -> 4.63, 40x256x36x36 14.1 -> 11.0 (5.3 TB/s),
+// 64x512x72x72 131 either way (5.5 TB/s).
+template <int VP, bool kDil>
+__global__ __launch_bounds__(256) void pack_dense_kernel(
+    const uint16_t* __restrict__ src, uint16_t* __restrict__ dst, int C, int H, int W, int S, int So,
+    int Wg, int wp, int lead, int chunks, int groups, int R, int ybl, int nimg, int64_t tail0) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t tile[];
+  constexpr int kVpShift = VP == 4 ? 2 : 0;
+  int bid = blockIdx.x;
+  const int64_t group_stride = int64_t(chunks) * kGroupRows * kKStep;
+  if (bid >= nimg) {
+    // rows [tail0, end) hold no image: zeros for every chunk
+    const int64_t phi = int64_t(groups) * kGroupOutRows + (kGroupRows - kGroupOutRows);
+    const int64_t n = (phi - tail0) * chunks * 8;
+    const uint4 z = make_uint4(0, 0, 0, 0);
+    for (int64_t i = int64_t(bid - nimg) * 256 + threadIdx.x; i < n; i += int64_t(gridDim.x - nimg) * 256) {
+      const int q = int(i & 7);
+      const int64_t rc = i >> 3;
+      const int chunk = int(rc % chunks);
+      put_row_piece(dst, tail0 + rc / chunks, q, z, chunks, chunk, groups);
+    }
+    return;
+  }
+  const int yb = bid % ybl;
+  bid /= ybl;
+  const int chunk = bid % chunks;
+  const int b = bid / chunks;
+  const int cc = min(C - chunk * kKStep, kKStep);
+  const int y0 = yb * R;
+  const int rows = min(R, H - y0);
+  // source planes: H x W, or ceil(H/2) x ceil(W/2) spread over H x W (kDil)
+  const int Hs = kDil ? (H + 1) >> 1 : H, Ws = kDil ? (W + 1) >> 1 : W;
+  const int ys0 = kDil ? y0 >> 1 : y0;
+  const int npix = (kDil ? min((rows + 1) >> 1, Hs - ys0) : rows) * Ws;
+  const int64_t plane = int64_t(Hs) * Ws;
+  const uint16_t* sbase = src + (int64_t(b) * C + chunk * kKStep) * plane + int64_t(ys0) * Ws;
+  // phase 1: the tile's run of every channel -> tile[pix][c].  An item is VP consecutive
+  // pixels x 16 channels: 16 loads of VP pixels each (all issued before the first LDS
+  // write), then VP x two 16-byte LDS writes.
+  const int nseg16 = (cc + 15) >> 4;
+  const int ngrp = (npix + VP - 1) / VP;
+  const uint32_t mgrp = ngrp > 1 ? 0xFFFFFFFFu / uint32_t(ngrp) + 1 : 0;
+  for (int it = threadIdx.x; it < nseg16 * ngrp; it += 256) {
+    const int seg = ngrp > 1 ? fast_div(it, mgrp) : it;
+    const int pix0 = min((it - seg * ngrp) * VP, npix - VP);
+    const uint16_t* sp = sbase + pix0;
+    uint32_t d[16][(VP + 1) / 2];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const int c = min(seg * 16 + k, cc - 1);
+      if (VP == 4) {
+        const Pix4 t = *reinterpret_cast<const Pix4*>(sp + c * plane);
+        d[k][0] = t.lo;
+        d[k][VP == 4 ? 1 : 0] = t.hi;
+      } else {
+        d[k][0] = sp[c * plane];
+      }
+    }
+    if (seg * 16 + 16 > cc) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+        if (seg * 16 + k >= cc)
+#pragma unroll
+          for (int i = 0; i < (VP + 1) / 2; ++i) d[k][i] = 0;
+    }
+#pragma unroll
+    for (int i = 0; i < VP; ++i) {
+      // dword m of pixel i: channel 2m (low half) and channel 2m + 1 (high half)
+      uint32_t o[8];
+#pragma unroll
+      for (int m = 0; m < 8; ++m) {
+        const uint32_t x = d[2 * m][i >> 1], y = d[2 * m + 1][i >> 1];
+        // v_perm_b32 selector: bytes 0-3 come from the second operand, 4-7 from the first
+        o[m] = VP == 1 ? (x | (y << 16))
+                       : ((i & 1) ? __builtin_amdgcn_perm(y, x, 0x07060302u)
+                                  : __builtin_amdgcn_perm(y, x, 0x05040100u));
+      }
+      *reinterpret_cast<uint4*>(tile + tile_piece<kVpShift>(pix0 + i, 2 * seg)) = make_uint4(o[0], o[1], o[2], o[3]);
+      *reinterpret_cast<uint4*>(tile + tile_piece<kVpShift>(pix0 + i, 2 * seg + 1)) = make_uint4(o[4], o[5], o[6], o[7]);
+    }
+  }
+  __syncthreads();
+
+  // phase 2: grid rows y0+1 .. y0+rows (plus the top / bottom border row for the first /
+  // last tile) of every strip, all wp columns, all 64 channels: packed rows
+  // [first, first + n) of the strip's virtual image, in runs of whole rows
+  const int gy_lo = y0 == 0 ? 0 : y0 + 1;
+  const int gy_hi = y0 + rows == H ? H + 2 : y0 + rows + 1;
+  const int n = (gy_hi - gy_lo) * wp * 8;
+  const uint32_t mwp = 0xFFFFFFFFu / uint32_t(wp) + 1;  // wp >= 3
+  for (int s = 0; s < S; ++s) {
+    const int64_t first = ((int64_t(b) * S + s) * (H + 2) + gy_lo) * wp;
+    const int64_t g = first >> 11;
+    const int r0 = int(first & (kGroupOutRows - 1));
+    uint16_t* out = dst + g * group_stride + int64_t(chunk) * kGroupRows * kKStep;
+    const int x0 = (S == 1 ? 0 : s * So - 1) - lead;
+    for (int t = threadIdx.x; t < n; t += 256) {
+      const int q = t & 7;
+      const int row = t >> 3;
+      const int gr = fast_div(row, mwp), gx = row - gr * wp;
+      const int gy = gy_lo + gr;
+      const int j = gx - lead, x = x0 + gx;
+      const bool real = gy >= 1 && gy <= H && unsigned(j) < unsigned(Wg) && unsigned(x) < unsigned(W) && q * 8 < cc;
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (kDil) {
+        // image row gy - 1 and column x even: source pixel ((gy - 1) / 2, x / 2)
+        if (real && ((gy - 1) & 1) == 0 && (x & 1) == 0)
+          v = *reinterpret_cast<const uint4*>(tile + tile_piece<kVpShift>((((gy - 1) >> 1) - ys0) * Ws + (x >> 1), q));
+      } else if (real) {
+        v = *reinterpret_cast<const uint4*>(tile + tile_piece<kVpShift>((gy - 1 - y0) * W + x, q));
+      }
+      const int rr = r0 + row;
+      const int gi = rr >> 11, r = rr & (kGroupOutRows - 1);
+      uint16_t* d = out + gi * group_stride + r * kKStep + q * 8;
+      if (g + gi < groups) *reinterpret_cast<uint4*>(d) = v;
+      if (g + gi > 0 && r < kGroupRows - kGroupOutRows)
+        *reinterpret_cast<uint4*>(d - group_stride + kGroupOutRows * kKStep) = v;
     }
   }
 }
@@ -383,36 +474,37 @@ int pack_launch(const char* what, const uint16_t* src, uint16_t* dst, int B, int
     if (blocks == 0) return 0;
     // the tile: R rows of W pixels, or R / 2 source rows of ceil(W/2) (kDil)
     const size_t lds = (dil ? size_t(R / 2) * size_t((W + 1) / 2) : size_t(R) * W) * kLdsPitch * 2;
+    const dim3 grid{unsigned(blocks)};
+    hipStream_t st = as_stream(stream);
+    if (dense) {
+      // the shortest run is the last tile's
+      const int last = H - (ybl - 1) * R;
+      const int64_t shortest = dil ? int64_t((last + 1) / 2) * ((W + 1) / 2) : int64_t(last) * W;
+#define XDNA_PACK_DENSE(vp, dl)                                                                           \
+  pack_dense_kernel<vp, dl><<<grid, 256, lds, st>>>(src, dst, C, H, W, S, So, Wg, wp, lead, chunks, ng, R, \
+                                                    ybl, int(nimg), tail0)
+      if (shortest >= 4) {
+        if (dil) XDNA_PACK_DENSE(4, true);
+        else XDNA_PACK_DENSE(4, false);
+      } else {
+        if (dil) XDNA_PACK_DENSE(1, true);
+        else XDNA_PACK_DENSE(1, false);
+      }
+#undef XDNA_PACK_DENSE
+      return check_launch(what);
+    }
     // pixels per lane load: every channel run (plane offset + y0 * W) must keep the
     // alignment of the load for every tile row start; the last group of a run is cut
     // short by the tile's pixel count only, and runs are padded in LDS to the group size
-    // (kDil: source planes ceil(H/2) x ceil(W/2), R / 2 source rows per tile)
-    const int64_t Ws = dil ? (W + 1) / 2 : W;
-    const int64_t plane = dil ? int64_t((H + 1) / 2) * Ws : int64_t(H) * W;
-    const int64_t tile_src = dil ? int64_t(R / 2) * Ws : int64_t(R) * W;
-    const int64_t step = std::gcd<int64_t>(plane, tile_src);  // all run offsets are multiples
+    const int64_t step = std::gcd<int64_t>(int64_t(H) * W, int64_t(R) * W);  // all run offsets are multiples
     const uintptr_t sa = reinterpret_cast<uintptr_t>(src);
-    const int VP = (sa % 8 == 0 && step % 4 == 0 && tile_src % 4 == 0) ? 4
-                   : (sa % 4 == 0 && step % 2 == 0 && tile_src % 2 == 0) ? 2 : 1;
-    const dim3 grid{unsigned(blocks)};
-    hipStream_t st = as_stream(stream);
-#define XDNA_PACK_LAUNCH(vp, dn, ...)                                                             \
-  pack_rows_lds_kernel<vp, dn, ##__VA_ARGS__><<<grid, 256, lds, st>>>(src, dst, C, H, W, S, So, Wg, wp, lead,  \
-                                                      halo_zero, chunks, g0, ng, int(b0), plo, phi, R, ybl,   \
-                                                      int(nimg), tail0)
-    if (dil) {
-      if (VP == 4) XDNA_PACK_LAUNCH(4, true, true);
-      else if (VP == 2) XDNA_PACK_LAUNCH(2, true, true);
-      else XDNA_PACK_LAUNCH(1, true, true);
-    } else if (dense) {
-      if (VP == 4) XDNA_PACK_LAUNCH(4, true);
-      else if (VP == 2) XDNA_PACK_LAUNCH(2, true);
-      else XDNA_PACK_LAUNCH(1, true);
-    } else {
-      if (VP == 4) XDNA_PACK_LAUNCH(4, false);
-      else if (VP == 2) XDNA_PACK_LAUNCH(2, false);
-      else XDNA_PACK_LAUNCH(1, false);
-    }
+    const int VP = (sa % 8 == 0 && step % 4 == 0) ? 4 : (sa % 4 == 0 && step % 2 == 0) ? 2 : 1;
+#define XDNA_PACK_LAUNCH(vp)                                                                              \
+  pack_rows_lds_kernel<vp><<<grid, 256, lds, st>>>(src, dst, C, H, W, S, So, Wg, wp, lead, halo_zero, chunks, \
+                                                   g0, ng, int(b0), plo, phi, R, ybl)
+    if (VP == 4) XDNA_PACK_LAUNCH(4);
+    else if (VP == 2) XDNA_PACK_LAUNCH(2);
+    else XDNA_PACK_LAUNCH(1);
 #undef XDNA_PACK_LAUNCH
     return check_launch(what);
   }

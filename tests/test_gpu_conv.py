@@ -154,6 +154,28 @@ def test_layout_pack(hip, shape, layout):
     assert hip.xdna_conv3x3_layout_packed_bytes(B, Cin, H, W, 2) == 0
 
 
+# runs that end inside a 4-pixel group, runs shorter than one, channel counts that end inside
+# a 16-channel segment or a 64-channel chunk, rows that cross groups and strips
+PACK_EDGES = [(3, 48, 29, 43), (5, 65, 9, 9), (2, 17, 5, 3), (4, 3, 3, 1), (1, 1, 1, 1), (2, 33, 1, 2), (40, 16, 7, 37),
+              (1, 70, 2, 255), (3, 130, 13, 6)]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("shape", PACK_EDGES, ids=lambda s: "x".join(map(str, s)))
+def test_layout_pack_edges(hip, shape, layout, offset):
+    """The dense pack at the edges of its 4-pixel loads, from sources on and off a 4-byte
+    boundary, bit for bit against the host construction."""
+    B, C, H, W = shape
+    print(f"pack edges {shape} layout {layout} offset {offset}", flush=True)
+    x = oracle.rng_bf16(np.random.default_rng(B + C + W), shape)
+    flat = dev(np.concatenate([np.full(offset, 0x7FC0, np.uint16), x.reshape(-1)]))
+    n = hip.xdna_conv3x3_layout_packed_bytes(B, C, H, W, layout)
+    buf = dev(np.full((n // 2,), 0xBEEF, np.uint16))
+    assert hip.xdna_conv3x3_layout_pack_bf16(ptr(flat[offset:]), ptr(buf), B, C, H, W, layout, stream()) == 0
+    np.testing.assert_array_equal(host(buf).reshape(-1), layout_util.pack_expected(x, layout).reshape(-1))
+
+
 @pytest.mark.parametrize("variant", VARIANTS, indirect=True, ids=lambda v: f"v{v}")
 @pytest.mark.parametrize("shape", LAYOUT_SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_forward_tight_layout(hip, shape, variant):
