@@ -374,6 +374,11 @@ int xdna_conv3x3_layout_rows_bf16(const uint16_t* xp, const uint16_t* wt, const 
 int xdna_conv2d_fwd_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int B,
                          int Cin, int Cout, int H, int W, int KH, int KW, int sh, int sw, int ph, int pw,
                          void* stream);
+/* act: 0 none, 1 ReLU, applied to the fp32 sum before its one rounding (the bits of relu of
+ * xdna_conv2d_fwd_bf16's output). */
+int xdna_conv2d_fwd_act_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int B,
+                             int Cin, int Cout, int H, int W, int KH, int KW, int sh, int sw, int ph, int pw,
+                             int act, void* stream);
 int xdna_conv2d_dgrad_bf16(const uint16_t* dy, const uint16_t* w, uint16_t* dx, int B, int Cin, int Cout,
                            int H, int W, int KH, int KW, int sh, int sw, int ph, int pw, void* stream);
 int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t* gb, int B, int Cin,
@@ -381,7 +386,8 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
                            void* stream);
 
 /* Kernel selection of xdna_conv2d_fwd_bf16 / xdna_conv2d_dgrad_bf16, for measurements and
- * tests: 0 automatic (default: at stride 1 with at most 32 output and at least 16 input
+ * tests: 0 automatic (default: at stride 1 with few channels on one side, the kernels that put
+ * kernel columns beside those channels; else at stride 1 with at most 32 output and at least 16 input
  * channels of the direction, and a padded output width up to 128, the direct form, which stages the
  * input rows of 4 output rows in LDS as a zero-padded grid and reads every tap as a row
  * offset; else the gather GEMM), 1 the gather GEMM only.  No reference counterpart. */

@@ -130,6 +130,16 @@ __device__ inline __amdgpu_buffer_rsrc_t uniform_buffer_rsrc(const void* p, int 
                                            0x00020000);
 }
 
+// Four pixels of one channel: an 8-byte load at the alignment the plane offsets leave
+// (global loads take any 2-byte address on gfx950).
+struct __attribute__((packed, aligned(2))) Pix4 {
+  uint32_t lo, hi;
+};
+
+// n / d for n * d < 2^32 and d > 1, with m = 0xFFFFFFFF / d + 1: one multiply instead of
+// the ~20 instructions of a division by a run-time value.
+__device__ inline int fast_div(int n, uint32_t m) { return int(__umulhi(uint32_t(n), m)); }
+
 // Split-K partial sums: init + src[z * stride] + src[(z + step) * stride] + ... over
 // indices below n, added left to right in that order (the fixed association every
 // deterministic reduce here keeps), with eight loads issued before their sums: a loop of

@@ -18,6 +18,7 @@
 // gradient splits its pixel reduction over blockIdx.z into fp32 partials, summed in a
 // fixed order by a second kernel (deterministic).
 #include "common.h"
+#include "conv_few.h"
 #include "mfma.h"
 #include "../../include/xdna_hip.h"
 
@@ -38,7 +39,7 @@ struct GArgs {
   uint16_t* out;         // forward: y; dgrad: dx
   float* part;           // wgrad: [nsplit][M][N]
   int B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw, Ho, Wo;
-  int M, N, K, kt_per, nsplit;
+  int M, N, K, kt_per, nsplit, act;
   int x_bytes, w_bytes, dy_bytes;  // operand extents (each under 2^31 bytes)
 };
 
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(256) void conv_gather_kernel(GArgs a) {
           if (m >= a.M) continue;
           float v = acc[i][j][r];
           if (DIR == kGFwd && a.bias) v += bf16_to_f32(a.bias[m]);
-          o[int64_t(m) * plane] = f32_to_bf16(v);
+          o[int64_t(m) * plane] = f32_to_bf16(act_forward(a.act, 0.0f, v));
         }
     }
   }
@@ -654,7 +655,7 @@ struct DArgs {
   const uint16_t* wp;    // prepared [chunks][KH][wv * 256 vectors of 8]: rows (co, kx) of 32 ci
   const uint16_t* bias;  // [Cout] or null
   uint16_t* out;         // [B][Cout][Ho][Wo]
-  int B, Cin, Cout, H, W, KH, KW, ph, pw, Ho, Wo, Wp, chunks, nb, xpos, rtiles, wv;
+  int B, Cin, Cout, H, W, KH, KW, ph, pw, Ho, Wo, Wp, chunks, nb, xpos, rtiles, wv, act;
   int x_bytes;           // under 2^31
 };
 
@@ -799,7 +800,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (co < a.Cout) {
         float v = acc[j][r];
         if (a.bias) v += bf16_to_f32(a.bias[co]);
-        o[int64_t(co) * a.Ho * a.Wo] = f32_to_bf16(v);
+        o[int64_t(co) * a.Ho * a.Wo] = f32_to_bf16(act_forward(a.act, 0.0f, v));
       }
     }
   }
@@ -839,7 +840,7 @@ std::atomic<int> g_conv2d_variant{0};  // 0 automatic, 1 gather GEMM only
 // Runs the direct form (weights prepared into the cache allocator) or returns 1 when it
 // does not apply.
 int run_direct(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* out, int B, int Cin,
-               int Cout, int H, int W, int KH, int KW, int ph, int pw, int flip, hipStream_t st) {
+               int Cout, int H, int W, int KH, int KW, int ph, int pw, int flip, int act, hipStream_t st) {
   DArgs d{};
   if (g_conv2d_variant.load() == 1 || !direct_args(d, B, Cin, Cout, H, W, KH, KW, ph, pw)) return 1;
   d.x_bytes = int(int64_t(B) * Cin * H * W * 2);  // the callers' operands are under 2^30 elements
@@ -863,6 +864,7 @@ int run_direct(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint1
   if (!wp) return -1;
   direct_prep_kernel<<<unsigned(std::min<int64_t>(ceil_div(n, 256), 4096)), 256, 0, st>>>(w, wp, Cin, Cout, KH, KW,
                                                                                           flip, blk, n);
+  d.act = act;
   d.x = x;
   d.wp = wp;
   d.bias = bias;
@@ -898,7 +900,18 @@ extern "C" {
 int xdna_conv2d_fwd_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int B,
                          int Cin, int Cout, int H, int W, int KH, int KW, int sh, int sw, int ph, int pw,
                          void* stream) {
+  return xdna_conv2d_fwd_act_bf16(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw, 0, stream);
+}
+
+int xdna_conv2d_fwd_act_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int B,
+                             int Cin, int Cout, int H, int W, int KH, int KW, int sh, int sw, int ph, int pw,
+                             int act, void* stream) {
+  if (act < 0 || act > 1) {
+    set_error("xdna_conv2d_fwd_act_bf16: activation must be 0 or 1");
+    return -1;
+  }
   GArgs a{};
+  a.act = act;
   if (!gconv_args("xdna_conv2d_fwd_bf16", a, B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw)) return -1;
   a.x = x; a.w = w; a.bias = bias; a.out = y;
   a.M = Cout; a.N = B * a.Ho * a.Wo; a.K = Cin * KH * KW;
@@ -910,7 +923,11 @@ int xdna_conv2d_fwd_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* b
   a.kt_per = int(ceil_div(a.K, kGTK));
   if (!admit_launch("xdna_conv2d_fwd_bf16")) return -1;
   if (sh == 1 && sw == 1) {
-    const int rc = run_direct(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, ph, pw, 0, as_stream(stream));
+    if (g_conv2d_variant.load() == 0) {
+      const int rc = conv_few_fwd(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, ph, pw, 0, act, as_stream(stream));
+      if (rc <= 0) return rc;
+    }
+    const int rc = run_direct(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, ph, pw, 0, act, as_stream(stream));
     if (rc <= 0) return rc;
   }
   return launch_gather<kGFwd>(a, as_stream(stream));
@@ -928,7 +945,12 @@ int xdna_conv2d_dgrad_bf16(const uint16_t* dy, const uint16_t* w, uint16_t* dx, 
   if (sh == 1 && sw == 1 && ph <= KH - 1 && pw <= KW - 1) {
     // at stride 1 the input gradient is the forward conv of dy with the flipped,
     // transposed weights and padding K - 1 - p, which gives back H x W
-    const int rc = run_direct(dy, w, nullptr, dx, B, Cout, Cin, a.Ho, a.Wo, KH, KW, KH - 1 - ph, KW - 1 - pw, 1,
+    if (g_conv2d_variant.load() == 0) {
+      const int rc = conv_few_fwd(dy, w, nullptr, dx, B, Cout, Cin, a.Ho, a.Wo, KH, KW, KH - 1 - ph, KW - 1 - pw, 1, 0,
+                                  as_stream(stream));
+      if (rc <= 0) return rc;
+    }
+    const int rc = run_direct(dy, w, nullptr, dx, B, Cout, Cin, a.Ho, a.Wo, KH, KW, KH - 1 - ph, KW - 1 - pw, 1, 0,
                               as_stream(stream));
     if (rc <= 0) return rc;
   }
@@ -942,6 +964,11 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
   if (!gconv_args("xdna_conv2d_wgrad_bf16", a, B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw)) return -1;
   a.x = x; a.dy = dy;
   hipStream_t st = as_stream(stream);
+  if (!admit_launch("xdna_conv2d_wgrad_bf16")) return -1;
+  if (sh == 1 && sw == 1 && g_conv2d_variant.load() == 0) {
+    const int rc = conv_few_wgrad(x, dy, gw, gb, B, Cin, Cout, H, W, KH, KW, ph, pw, st);
+    if (rc <= 0) return rc;
+  }
   FsArgs fs{};
   int fs_nt = 0;
   if (slide_args(fs, B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw, a.Ho, a.Wo, fs_nt)) {
@@ -949,7 +976,6 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
     fs.dy = dy;
     const int64_t nwg = ceil_div(fs.rows, fs.rows_per_wg);
     const int64_t mn = int64_t(Cout) * Cin * KH * KW;
-    if (!admit_launch("xdna_conv2d_wgrad_bf16")) return -1;
     fs.part = static_cast<float*>(xdna_hip_cache_alloc(size_t(nwg) * size_t(mn) * sizeof(float)));
     if (!fs.part) return -1;
     const size_t lds = slide_lds(Cin, KH, fs.pitch, fs.R, fs.Wo);
@@ -977,7 +1003,6 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
     f.rows_per_wg = int(ceil_div(f.rows, wgs));
     const int64_t nwg = ceil_div(f.rows, f.rows_per_wg);
     const int64_t mn = int64_t(Cout) * Cin * KH * KW;
-    if (!admit_launch("xdna_conv2d_wgrad_bf16")) return -1;
     f.part = static_cast<float*>(xdna_hip_cache_alloc(size_t(nwg) * size_t(mn) * sizeof(float)));
     if (!f.part) return -1;
     const size_t lds = size_t(int64_t(Cin) * KH * f.Wp + 4 * f.Wo) * 4;
@@ -1001,7 +1026,6 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
   a.kt_per = int(ceil_div(ktiles, ns));
   a.nsplit = int(ceil_div(ktiles, a.kt_per));
   const int64_t mn = int64_t(a.M) * a.N;
-  if (!admit_launch("xdna_conv2d_wgrad_bf16")) return -1;
   a.part = static_cast<float*>(xdna_hip_cache_alloc(size_t(a.nsplit) * size_t(mn) * sizeof(float)));
   if (!a.part) return -1;
   if (launch_gather<kGWgrad>(a, st)) {

@@ -222,16 +222,6 @@ __global__ __launch_bounds__(256) void pack_rows_lds_kernel(
   }
 }
 
-// Four pixels of one channel: an 8-byte load at the alignment the plane offsets leave
-// (global loads take any 2-byte address on gfx950).
-struct __attribute__((packed, aligned(2))) Pix4 {
-  uint32_t lo, hi;
-};
-
-// n / d for n * d < 2^32 and d > 1, with m = 0xFFFFFFFF / d + 1: one multiply instead of
-// the ~20 instructions of a division by a run-time value.
-__device__ inline int fast_div(int n, uint32_t m) { return int(__umulhi(uint32_t(n), m)); }
-
 // The dense pack of the conv path: every element of every group is written, zeros included
 // (border rows and columns, padded channels, the rows past the last image), so a buffer
 // needs no fill; workgroups from nimg on write the rows past the last image.

@@ -823,12 +823,21 @@ bool gconv_auto(int cout, int sh, int sw) { return cout >= 32 && sh == 1 && sw =
 // 3x3 / stride-1 convs with at most 4 input channels (RGB input layers): the rows path
 // pads the input to a 64-channel chunk (16-21x the MACs), so their forward and weight
 // gradient take the general kernels (measured on MI355X: ResNet-18's stem B128 3->64 at
-// 64x64 forward 80.6 -> 31.0 us, weight gradient 209 -> 133 us; VGG's first layer B40 at
-// 36x36 forward 19.2 -> 8.5 us); their input gradient (64 input channels of the gradient
-// conv) stays on the rows path, which is faster there.
+// 64x64 forward 80.6 -> 30.3 us, weight gradient 209 -> 76 us; VGG's first layer B40 at
+// 36x36 forward 19.2 -> 7.2 us).  So does their input gradient where the few-channel form
+// fits (few_input_dx): VGG's first layer 13.3 (pack and rows conv) -> 9.8 us.
 bool few_input_3x3(const at::Tensor& x, const at::Tensor& w) {
   const int m = g_gconv_mode.load();
   return x.size(1) <= 4 && (m == 2 || (m == 1 && gconv_auto(int(w.size(0)), 1, 1)));
+}
+// the general kernels' operand limits for a 3x3 / stride-1 / pad-1 layer
+bool gconv_fits_3x3(const at::Tensor& x, const at::Tensor& w) {
+  const int64_t pixels = x.size(0) * x.size(2) * x.size(3);
+  return pixels > 0 && pixels * std::max(x.size(1), w.size(0)) < (int64_t(1) << 30);
+}
+bool few_input_dx(const at::Tensor& x, const at::Tensor& w) {
+  return g_gconv_mode.load() == 2 && !g_bfp16_emul.load() && w.size(0) >= 8 && x.size(3) >= 4 && x.size(3) <= 256 &&
+         gconv_fits_3x3(x, w);
 }
 bool gconv_auto_fwd(int cin, int cout, int sh, int sw) {
   return gconv_auto(cout, sh, sw) || (cout <= 32 && cin >= 16 && sh == 1 && sw == 1);
@@ -853,20 +862,32 @@ GeomArgs gconv_geom(const at::Tensor& x, const at::Tensor& w, c10::SymIntArrayRe
 }
 
 at::Tensor hip_gconv_fwd(const at::Tensor& input, const at::Tensor& weight, const at::Tensor* bias,
-                         c10::SymIntArrayRef stride, c10::SymIntArrayRef padding) {
+                         c10::SymIntArrayRef stride, c10::SymIntArrayRef padding, int act = 0) {
   const GeomArgs g = gconv_geom(input, weight, stride, padding);
   at::Tensor x = input.contiguous(), w = weight.contiguous();
   at::Tensor bc;
   if (bias) bc = bias->contiguous();
   at::Tensor y = empty_xdna({g.B, g.Cout, g.Ho, g.Wo}, at::kBFloat16);
   KernelTimer kt("conv2d.fwd", 2.0 * g.B * g.Ho * g.Wo * double(g.Cout) * g.Cin * g.KH * g.KW);
-  check_abi(xdna_conv2d_fwd_bf16(static_cast<const uint16_t*>(x.const_data_ptr()),
-                                 static_cast<const uint16_t*>(w.const_data_ptr()),
-                                 bias ? static_cast<const uint16_t*>(bc.const_data_ptr()) : nullptr,
-                                 static_cast<uint16_t*>(y.data_ptr()), g.B, g.Cin, g.Cout, g.H, g.W, g.KH,
-                                 g.KW, g.sh, g.sw, g.ph, g.pw, current_stream()),
+  check_abi(xdna_conv2d_fwd_act_bf16(static_cast<const uint16_t*>(x.const_data_ptr()),
+                                     static_cast<const uint16_t*>(w.const_data_ptr()),
+                                     bias ? static_cast<const uint16_t*>(bc.const_data_ptr()) : nullptr,
+                                     static_cast<uint16_t*>(y.data_ptr()), g.B, g.Cin, g.Cout, g.H, g.W, g.KH,
+                                     g.KW, g.sh, g.sw, g.ph, g.pw, act, current_stream()),
             "conv2d forward");
   return y;
+}
+
+at::Tensor hip_gconv_dgrad(const at::Tensor& grad, const at::Tensor& weight, const GeomArgs& g) {
+  at::Tensor d = grad.contiguous(), w = weight.contiguous();
+  at::Tensor dx = empty_xdna({g.B, g.Cin, g.H, g.W}, at::kBFloat16);
+  KernelTimer kt("conv2d.dgrad", 2.0 * g.B * g.Ho * g.Wo * double(g.Cout) * g.Cin * g.KH * g.KW);
+  check_abi(xdna_conv2d_dgrad_bf16(static_cast<const uint16_t*>(d.const_data_ptr()),
+                                   static_cast<const uint16_t*>(w.const_data_ptr()),
+                                   static_cast<uint16_t*>(dx.data_ptr()), g.B, g.Cin, g.Cout, g.H, g.W, g.KH, g.KW,
+                                   g.sh, g.sw, g.ph, g.pw, current_stream()),
+            "conv2d dgrad");
+  return dx;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1163,9 +1184,10 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
   // dY packed once: the input gradient's conv and the rows weight gradient read it
   const int layout = g_conv_layout.load();
   at::Tensor gop;
+  const bool dx_few = few_in && mask[0] && few_input_dx(input, weight);
   // the input gradient alone reads dY: a small grid reads it in place
-  const bool dx_nchw = hip && mask[0] && !dw_rows && !strided && nchw_route(go, weight.size(1), true);
-  if (hip && ((mask[0] && !dx_nchw) || dw_rows))
+  const bool dx_nchw = hip && mask[0] && !dx_few && !dw_rows && !strided && nchw_route(go, weight.size(1), true);
+  if (hip && ((mask[0] && !dx_nchw && !dx_few) || dw_rows))
     gop = strided ? pack_rows_spread(grad_output, go_sizes[2], go_sizes[3], layout) : pack_rows(go, layout);
   // the rows weight gradient beside the input gradient (captured graphs only)
   const bool both = dw_rows && mask[0];
@@ -1179,8 +1201,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
   }
   if (hip && mask[0]) {
     ScopedCount sc("hip_conv3x3.dx.run");
-    gi = dx_nchw ? hip_conv_nchw(go, weight, nullptr, true)
-                 : hip_conv_packed(gop, layout, go_sizes, weight, nullptr, true, 0, !strided);
+    gi = dx_few    ? hip_gconv_dgrad(go, weight, gconv_geom(input, weight, stride, padding))
+         : dx_nchw ? hip_conv_nchw(go, weight, nullptr, true)
+                   : hip_conv_packed(gop, layout, go_sizes, weight, nullptr, true, 0, !strided);
     mask[0] = false;
   }
   if (strided && dw && !dw_rows) {
@@ -1251,14 +1274,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
     const bool auto_ok = gconv_auto(g.Cout, g.sh, g.sw);
     if (mask[0] && (gmode == 2 || gconv_auto_dgrad(g))) {
       ScopedCount sc("hip_conv2d.dx.run");
-      at::Tensor w = weight.contiguous();
-      gi = empty_xdna({g.B, g.Cin, g.H, g.W}, at::kBFloat16);
-      KernelTimer kt("conv2d.dgrad", flops);
-      check_abi(xdna_conv2d_dgrad_bf16(static_cast<const uint16_t*>(d.const_data_ptr()),
-                                       static_cast<const uint16_t*>(w.const_data_ptr()),
-                                       static_cast<uint16_t*>(gi.data_ptr()), g.B, g.Cin, g.Cout, g.H, g.W,
-                                       g.KH, g.KW, g.sh, g.sw, g.ph, g.pw, current_stream()),
-                "conv2d dgrad");
+      gi = hip_gconv_dgrad(d, weight, g);
       mask[0] = false;
     }
     if (mask[1] && g_mode.load() >= 2 && (gmode == 2 || auto_ok)) {
@@ -2245,6 +2261,10 @@ at::Tensor region_conv3x3(const at::Tensor& x, const at::Tensor& w, const std::o
                     b->device().type() == kXdna,
                 "region conv: bias must be a bf16 xdna vector of the output channels");
   ScopedCount sc(act ? "hip_region.conv_relu.run" : "hip_region.conv.run");
+  if (few_input_3x3(x, w) && !g_bfp16_emul.load() && gconv_fits_3x3(x, w)) {
+    const c10::SymInt one[2] = {1, 1};
+    return hip_gconv_fwd(x, w, has_b ? &*b : nullptr, one, one, act);
+  }
   if (nchw_route(x, w.size(0), true)) return hip_conv_nchw(x, w, has_b ? &*b : nullptr, false, act);
   const int layout = g_conv_layout.load();
   return hip_conv_packed(pack_rows(x, layout), layout, x.sizes(), w, has_b ? &*b : nullptr, false, act);

@@ -84,6 +84,7 @@ SIGNATURES = {
     "xdna_instance_norm_act_fwd_bf16": (I, [P, P, P, I, P, P, P, L, L, L, D, I, F, P]),
     "xdna_instance_norm_act_bwd_bf16": (I, [P, P, P, P, I, P, P, P, P, P, L, L, L, I, F, P]),
     "xdna_upsample_nearest2x_bf16": (I, [P, P, L, I, I, P]),
+    "xdna_conv2d_fwd_act_bf16": (I, [P, P, P, P] + [I] * 12 + [P]),
     "xdna_conv2d_set_variant": (I, [I]),
     "xdna_subsample2_bf16": (I, [P, P, L, I, I, P]),
     "xdna_conv3x3_prepare_weights_both_bf16": (I, [P, P, P, I, I, P]),

@@ -102,6 +102,65 @@ def test_wgrad(hip, case):
     np.testing.assert_array_equal(host(gw2), got)
 
 
+# stride-1 layers with few channels on one side (taps beside the few channels): k pads, tile
+# and channel remainders, one few channel and four, paddings from none to the full kernel,
+# rows from 4 columns to ones that leave no room for a second workgroup
+FEW = [
+    (3, 8, 1, 5, 4, 3, 3, 1, 1, 1, 1), (2, 33, 3, 13, 11, 9, 9, 1, 1, 4, 4), (2, 70, 4, 9, 30, 5, 7, 1, 1, 2, 3),
+    (2, 3, 70, 13, 17, 9, 9, 1, 1, 4, 4), (3, 1, 40, 7, 9, 5, 3, 1, 1, 0, 0), (2, 4, 33, 12, 20, 3, 5, 1, 1, 2, 4),
+    (1, 2, 9, 6, 130, 7, 7, 1, 1, 3, 3), (1, 40, 3, 6, 150, 9, 9, 1, 1, 4, 4), (2, 32, 3, 16, 10, 1, 9, 1, 1, 0, 8),
+    (5, 3, 64, 20, 27, 3, 3, 1, 1, 1, 1), (2, 9, 2, 11, 12, 16, 9, 1, 1, 8, 4), (700, 3, 16, 4, 4, 3, 3, 1, 1, 1, 1),
+]
+
+
+@pytest.mark.parametrize("case", FEW, ids=lambda c: "x".join(map(str, c)))
+def test_few_channels(hip, case):
+    B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw = case
+    print(f"conv2d few channels {case}", flush=True)
+    x, w, b, dy, Ho, Wo = _data(case, sum(case) + 3)
+    y, dx = dev_zeros((B, Cout, Ho, Wo)), dev_zeros((B, Cin, H, W))
+    gw, gb = dev_zeros((Cout, Cin, KH, KW)), dev_zeros((Cout,))
+    d = (B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw, stream())
+    xd, wd, dyd = dev(x), dev(w), dev(dy)
+    assert hip.xdna_conv2d_fwd_bf16(ptr(xd), ptr(wd), ptr(dev(b)), ptr(y), *d) == 0
+    check_bf16(host(y), oracle.conv2d_fwd(x, w, b, (sh, sw), (ph, pw)), what=f"fwd {case}")
+    assert hip.xdna_conv2d_dgrad_bf16(ptr(dyd), ptr(wd), ptr(dx), *d) == 0
+    check_bf16(host(dx), oracle.conv2d_dgrad(dy, w, (H, W), (sh, sw), (ph, pw)), what=f"dgrad {case}")
+    assert hip.xdna_conv2d_wgrad_bf16(ptr(xd), ptr(dyd), ptr(gw), ptr(gb), *d) == 0
+    ref_w, ref_b = oracle.conv2d_wgrad(x, dy, (KH, KW), (sh, sw), (ph, pw))
+    check_bf16(host(gw), ref_w, what=f"wgrad {case}")
+    check_bf16(host(gb), ref_b, what=f"bias grad {case}")
+
+
+@pytest.mark.parametrize("cin,cout", [(12, 3), (3, 12)])
+def test_few_channels_keep_infinities_in_their_pairs(hip, cin, cout):
+    """An infinity in x reaches the outputs whose window holds it and the weight gradients of
+    its own channel, and nothing else (the kernels multiply padding beside it)."""
+    B, H, W, K, p = 2, 9, 13, 9, 4
+    rng = np.random.default_rng(cin)
+    xf = rng.standard_normal((B, cin, H, W)).astype(np.float32)
+    xf[1, 2, 0, W - 1] = np.inf
+    x = oracle.bf16_bits(xf)
+    w = oracle.bf16_bits(rng.uniform(0.1, 1, (cout, cin, K, K)).astype(np.float32))
+    dy = oracle.bf16_bits(rng.uniform(0.1, 1, (B, cout, H, W)).astype(np.float32))
+    y, gw = dev_zeros((B, cout, H, W)), dev_zeros((cout, cin, K, K))
+    d = (B, cin, cout, H, W, K, K, 1, 1, p, p, stream())
+    print(f"few channels with an infinity {cin} -> {cout}", flush=True)
+    assert hip.xdna_conv2d_fwd_bf16(ptr(dev(x)), ptr(dev(w)), None, ptr(y), *d) == 0
+    assert hip.xdna_conv2d_wgrad_bf16(ptr(dev(x)), ptr(dev(dy)), ptr(gw), None, *d) == 0
+    finite = np.ones((B, cout, H, W), bool)
+    finite[1, :, :p + 1, W - 1 - p:] = False
+    np.testing.assert_array_equal(np.isfinite(oracle.bf16_value(host(y))), finite)
+    # tap (ky, kx) pairs x[0][W - 1] with dy[p - ky][W - 1 + p - kx] where that exists
+    finite = np.ones((cout, cin, K, K), bool)
+    finite[:, 2, :p + 1, p:] = False
+    got = oracle.bf16_value(host(gw))
+    np.testing.assert_array_equal(np.isfinite(got), finite)
+    xf[1, 2, 0, W - 1] = 0
+    ref, _ = oracle.conv2d_wgrad(oracle.bf16_bits(xf), dy, (K, K), (1, 1), (p, p))
+    check_bf16(np.where(finite, host(gw), 0), np.where(finite, ref, 0), what="weight gradient beside an infinity")
+
+
 def test_invalid_shapes(hip):
     y = dev_zeros((1,))
     assert hip.xdna_conv2d_fwd_bf16(ptr(y), ptr(y), None, ptr(y), 1, 1, 1, 2, 2, 5, 5, 1, 1, 0, 0, stream()) == -1
