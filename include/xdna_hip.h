@@ -361,6 +361,28 @@ int xdna_conv3x3_layout_pack_bf16(const uint16_t* src, uint16_t* dst, int B, int
 int xdna_conv3x3_layout_rows_bf16(const uint16_t* xp, const uint16_t* wt, const uint16_t* bias, uint16_t* y,
                                   int B, int cin, int cout, int H, int W, int layout, void* stream);
 
+/* The same convs as implicit GEMMs over real output pixels (no border rows, native strides).
+ * H x W is the stride-1 image.  form 0: 3x3 / stride 1 / pad 1 from the packed rows of x; 1: the
+ * forward of 3x3 / stride 2 / pad 1 (y ceil(H/2) x ceil(W/2)) from the packed rows of x; 2: that
+ * conv's input gradient (y H x W) from the packed rows of the ceil(H/2) x ceil(W/2) gradient and
+ * the input gradient's prepared weights, cin and cout being the gradient's and x's channels.
+ * act as above; tile 0 automatic (others for measurements).  Returns -1 for operands past
+ * 32-bit offsets. */
+int xdna_conv3x3_px_bf16(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bias, uint16_t* y, int B,
+                         int cin, int cout, int H, int W, int layout, int act, int tile, void* stream);
+
+/* Whether these kernels are the better choice (and take the operands): op 0 stride-1 conv, 1
+ * stride-2 forward, 2 stride-2 input gradient, 3 stride-1 weight gradient, 4 stride-2 weight
+ * gradient.  0 where a kernel of the rows or weight-gradient forms is forced. */
+int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int layout);
+/* Their weight gradient (form 0 or 1; + bias gradient when gb is not null) from the packed rows
+ * of x (H x W) and of the conv's output gradient; the pixel reduction is split over workgroups
+ * and summed in a fixed order. */
+size_t xdna_conv3x3_px_wgrad_workspace_bytes(int form, int B, int Cin, int Cout, int H, int W);
+int xdna_conv3x3_px_wgrad_bf16(int form, const uint16_t* xp, const uint16_t* dp, uint16_t* gw, uint16_t* gb, int B,
+                               int Cin, int Cout, int H, int W, int layout, void* workspace, size_t workspace_bytes,
+                               void* stream);
+
 /* General 2-D convolution, bf16 in/out, fp32 accumulation: any kernel size, stride and
  * padding (dilation 1, groups 1), NCHW activations and OIHW weights.  Replaces the
  * reference's CPU route for convolutions outside its 3x3 path

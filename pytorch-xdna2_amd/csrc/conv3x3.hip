@@ -27,6 +27,7 @@
 // every call returns the same bits.  The bias gradient rides along in the
 // first channel tile.
 #include "common.h"
+#include "conv_px.h"
 #include "mfma.h"
 #include "../../include/xdna_hip.h"
 
@@ -3108,10 +3109,11 @@ void wgrad_rows5_kernel(WgRowsArgs a) {
 // The default, form 2: 2.2 % ahead of form 1 over the sweep's 36 shapes (GPU time per
 // shape's fwd + dgrad + wgrad step), 3 % on the largest ones.
 constexpr int kWgradRowsDefaultForm = 2;
+// (0: not forced)
 std::atomic<int> g_wgrad_rows_form{[] {
   const char* e = std::getenv("XDNA_WGRAD_KERNEL");
   const int f = e ? std::atoi(e) : 0;
-  return f == 1 || f == 2 ? f : kWgradRowsDefaultForm;
+  return f == 1 || f == 2 ? f : 0;
 }()};
 
 struct WgRowsPlan {
@@ -3137,7 +3139,7 @@ WgRowsPlan wgrad_rows_plan(int B, int Cin, int Cout, int H, int W, int layout) {
   p.ci_chunks = int(ceil_div(Cin, kKStep));
   p.co_chunks = int(ceil_div(Cout, kKStep));
   p.ci_pad = p.ci_chunks * kKStep;
-  p.form = g_wgrad_rows_form.load();
+  p.form = g_wgrad_rows_form.load() ? g_wgrad_rows_form.load() : kWgradRowsDefaultForm;
   {
     // form 2's tile (xdna_conv3x3_set_wgrad_tile forces one): four waves on 64 output
     // channels for layers of up to 64 output channels and for layers of up to 256 channels
@@ -3506,6 +3508,71 @@ int xdna_conv3x3_layout_rows_stride2_bf16(const uint16_t* xp, const uint16_t* wt
   return launch_rows(xp, wt, bias, y, B, cin, cout, H, W, stream, layout, 0, /*s2out=*/true);
 }
 
+int xdna_conv3x3_px_bf16(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bias, uint16_t* y, int B,
+                         int cin, int cout, int H, int W, int layout, int act, int tile, void* stream) {
+  if (!shape_ok("xdna_conv3x3_px_bf16", B, cin, cout, H, W)) return -1;
+  if (form < kPxStride1 || form > kPxS2Dgrad || (layout != kLayoutRef && layout != kLayoutTight) || act < 0 ||
+      act > 1 || !conv_px_fits(form, B, cin, cout, H, W, layout)) {
+    set_error("xdna_conv3x3_px_bf16: unknown form, layout or activation, or operands too large");
+    return -1;
+  }
+  if (!admit_launch("xdna_conv3x3_px_bf16")) return -1;
+  return conv_px(form, xp, wt, bias, y, B, cin, cout, H, W, layout, act, tile, as_stream(stream));
+}
+
+int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int layout) {
+  if (B < 1 || cin < 1 || cout < 1 || H < 1 || W < 1 || (layout != kLayoutRef && layout != kLayoutTight)) return 0;
+  if (op < 3 && g_rows_variant.load() != 0) return 0;
+  if (op >= 3 && (g_wgrad_rows_form.load() != 0 || g_wgrad_tile.load() != 0)) return 0;
+  const int form = op == 0 || op == 3 ? kPxStride1 : op == 2 ? kPxS2Dgrad : kPxStride2;
+  if (op < 0 || op > 4 || !conv_px_fits(form, B, cin, cout, H, W, layout)) return 0;
+  // (the weight gradient reads dY's packed rows, too)
+  if (op >= 3 && !conv_px_fits(kPxStride1, B, cout, cin, H, W, layout)) return 0;
+  if (op == 1 || op == 2 || op == 4) return 1;
+  if (op == 0) {
+    // grids the window kernels leave to their small-grid form, from 256 input channels: 256ch
+    // 40 x 9 x 9 13.4 -> 12.5 us (and 16.1 with the pack, where the form reading NCHW in place
+    // takes 19.3), 512 -> 256 at 40 x 4 x 4 16.8 -> 11.4 (23.1 in place); with fewer chunks the
+    // window's reuse by its nine taps is worth more (128ch 40 x 9 x 9 7.0 against 10.1)
+    const ConvGeom g = conv_geom(B, H, W, layout);
+    return cin > 3 * kKStep && ceil_div(g.m_total, 256) * ceil_div(cout, kSCo) < 150;
+  }
+  // the weight gradient: up to 30 GFLOP (128ch 40 x 36 x 36 36.4 -> 29.9 us, 40 x 9 x 9 20.2 ->
+  // 15.9, 512ch 16 x 18 x 18 52.9 -> 45.0; beyond, 128ch 128 x 32 x 32 60.6 against 63), on one
+  // chunk of input channels (64ch 128 x 64 x 64 64.2 -> 57.1) and on images whose padded grid
+  // is half border (512ch 128 x 8 x 8 69.5 -> 56.7)
+  const double gflop = 2.0 * 9.0 * double(B) * H * W * double(cin) * double(cout) * 1e-9;
+  return cin <= kKStep || gflop <= 30.0 || H * W <= 64;
+}
+
+size_t xdna_conv3x3_px_wgrad_workspace_bytes(int form, int B, int Cin, int Cout, int H, int W) {
+  if (B < 1 || Cin < 1 || Cout < 1 || H < 1 || W < 1 || (form != kPxStride1 && form != kPxStride2)) return 0;
+  const PxWgradPlan p = conv_px_wgrad_plan(form, B, Cin, Cout, H, W, g_wgrad_splits.load());
+  return align256(p.part_bytes) + align256(p.bpart_bytes);
+}
+
+int xdna_conv3x3_px_wgrad_bf16(int form, const uint16_t* xp, const uint16_t* dp, uint16_t* gw, uint16_t* gb, int B,
+                               int Cin, int Cout, int H, int W, int layout, void* workspace, size_t workspace_bytes,
+                               void* stream) {
+  if (!shape_ok("xdna_conv3x3_px_wgrad_bf16", B, Cin, Cout, H, W)) return -1;
+  if ((form != kPxStride1 && form != kPxStride2) || (layout != kLayoutRef && layout != kLayoutTight) ||
+      !conv_px_fits(form, B, Cin, Cout, H, W, layout) || !conv_px_fits(kPxStride1, B, Cout, Cin, H, W, layout)) {
+    set_error("xdna_conv3x3_px_wgrad_bf16: unknown form or layout, or operands too large");
+    return -1;
+  }
+  const PxWgradPlan p = conv_px_wgrad_plan(form, B, Cin, Cout, H, W, g_wgrad_splits.load());
+  if (!workspace || workspace_bytes < align256(p.part_bytes) + align256(p.bpart_bytes)) {
+    set_error("xdna_conv3x3_px_wgrad_bf16: workspace too small");
+    return -1;
+  }
+  if (!admit_launch("xdna_conv3x3_px_wgrad_bf16")) return -1;
+  float* part = static_cast<float*>(workspace);
+  float* bpart = gb ? reinterpret_cast<float*>(static_cast<char*>(workspace) + align256(p.part_bytes)) : nullptr;
+  if (conv_px_wgrad(p, form, xp, dp, part, bpart, B, Cin, Cout, H, W, layout, as_stream(stream))) return -1;
+  launch_wgrad_reduce(part, bpart, gw, gb, Cout, Cin, p.co_pad, p.ci_pad, p.splits, as_stream(stream));
+  return check_launch("xdna_conv3x3_px_wgrad_bf16");
+}
+
 int xdna_conv3x3_layout_rows_bfp16_emul_bf16(const uint16_t* xp, const uint16_t* wt, const uint16_t* bias,
                                              uint16_t* y, int B, int cin, int cout, int H, int W, int layout, int act,
                                              void* stream) {
@@ -3535,7 +3602,7 @@ int xdna_conv3x3_set_wgrad_rows_kernel(int form) {
     set_error("xdna_conv3x3_set_wgrad_rows_kernel: form must be 0 (default), 1 or 2");
     return -1;
   }
-  g_wgrad_rows_form.store(form == 0 ? kWgradRowsDefaultForm : form);
+  g_wgrad_rows_form.store(form);
   return 0;
 }
 

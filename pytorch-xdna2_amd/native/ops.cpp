@@ -521,8 +521,16 @@ std::atomic<int> g_conv_nchw{[] {
   return e && std::atoi(e) == 0 ? 0 : 1;
 }()};
 
+// Where the real-pixel kernels are the better choice (xdna_conv3x3_px_pick's ops), for a conv
+// of the H x W image sizes[2] x sizes[3].
+enum PxOp { kPxFwd = 0, kPxS2Fwd = 1, kPxS2Dx = 2, kPxDw = 3, kPxS2Dw = 4 };
+bool px_pick(PxOp op, at::IntArrayRef sizes, int64_t cin, int64_t cout, int layout) {
+  return xdna_conv3x3_px_pick(op, int(sizes[0]), int(cin), int(cout), int(sizes[2]), int(sizes[3]), layout) == 1;
+}
+
 bool nchw_route(const at::Tensor& src, int64_t cout, bool s1) {
   if (!g_conv_nchw.load() || (s1 && g_bfp16_emul.load())) return false;
+  if (px_pick(s1 ? kPxFwd : kPxS2Fwd, src.sizes(), src.size(1), cout, g_conv_layout.load())) return false;
   return xdna_conv3x3_nchw_small_eligible(int(src.size(0)), int(src.size(1)), int(cout), int(src.size(2)),
                                           int(src.size(3))) == 1;
 }
@@ -561,8 +569,20 @@ at::Tensor hip_conv_packed(const at::Tensor& packed, int layout, at::IntArrayRef
   at::Tensor bc;
   if (bias) bc = bias->contiguous();
   const double flops = 2.0 * double(B) * double(H) * double(W) * double(cin) * double(cout) * 9.0;
+  const auto px = [&](int form) {
+    check_abi(xdna_conv3x3_px_bf16(form, static_cast<const uint16_t*>(packed.const_data_ptr()),
+                                   static_cast<const uint16_t*>(wt.const_data_ptr()),
+                                   bias ? static_cast<const uint16_t*>(bc.const_data_ptr()) : nullptr,
+                                   static_cast<uint16_t*>(out.data_ptr()), int(B), int(cin), int(cout), int(H), int(W),
+                                   layout, act, 0, st),
+              "conv pixels");
+  };
   if (s2out) {
     KernelTimer kt("conv3x3_rows.s2", flops);
+    if (px_pick(kPxS2Fwd, src, cin, cout, layout)) {
+      px(kPxS2Fwd);
+      return out;
+    }
     check_abi(xdna_conv3x3_layout_rows_stride2_bf16(
                   static_cast<const uint16_t*>(packed.const_data_ptr()), static_cast<const uint16_t*>(wt.const_data_ptr()),
                   bias ? static_cast<const uint16_t*>(bc.const_data_ptr()) : nullptr,
@@ -580,6 +600,10 @@ at::Tensor hip_conv_packed(const at::Tensor& packed, int layout, at::IntArrayRef
     return out;
   }
   KernelTimer kt(dgrad ? "conv3x3_rows.dgrad" : "conv3x3_rows.fwd", flops);
+  if (s1 && px_pick(kPxFwd, src, cin, cout, layout)) {
+    px(kPxFwd);
+    return out;
+  }
   check_abi(xdna_conv3x3_layout_rows_act_bf16(static_cast<const uint16_t*>(packed.const_data_ptr()),
                                               static_cast<const uint16_t*>(wt.const_data_ptr()),
                                               bias ? static_cast<const uint16_t*>(bc.const_data_ptr()) : nullptr,
@@ -587,6 +611,20 @@ at::Tensor hip_conv_packed(const at::Tensor& packed, int layout, at::IntArrayRef
                                               int(H), int(W), layout, act, st),
             "conv rows");
   return out;
+}
+
+// The input gradient of a 3x3 / stride-2 / pad-1 conv with weight w, into sizes, from the
+// packed rows of its output gradient.
+at::Tensor hip_conv_s2_dx(const at::Tensor& dpacked, int layout, at::IntArrayRef sizes, const at::Tensor& w) {
+  at::Tensor wt = conv_weight_form(w, true);
+  at::Tensor dx = empty_xdna(sizes, at::kBFloat16);
+  KernelTimer kt("conv3x3_rows.dgrad", 2.0 * double(dx.numel()) * double(w.size(0)) * 9.0 / 4.0);
+  check_abi(xdna_conv3x3_px_bf16(kPxS2Dx, static_cast<const uint16_t*>(dpacked.const_data_ptr()),
+                                 static_cast<const uint16_t*>(wt.const_data_ptr()), nullptr,
+                                 static_cast<uint16_t*>(dx.data_ptr()), int(sizes[0]), int(w.size(0)), int(w.size(1)),
+                                 int(sizes[2]), int(sizes[3]), layout, 0, 0, current_stream()),
+            "conv stride-2 input gradient");
+  return dx;
 }
 
 at::Tensor hip_conv(const at::Tensor& src, const at::Tensor& w, const at::Tensor* bias, bool dgrad) {
@@ -1066,9 +1104,13 @@ struct WgradRowsJob {
   size_t wsb = 0;
   int64_t B = 0, Cin = 0, Cout = 0, H = 0, W = 0;
   int layout = 0;
+  int px = -1;  // form of the real-pixel kernel (0 stride 1, 1 stride 2), -1: the window kernels
 };
 
-WgradRowsJob wgrad_rows_prepare(const at::Tensor& input, int layout, int64_t Cout, at::Tensor& gw, at::Tensor* gb) {
+// stride: the conv's; px2: a stride-2 conv whose dY is packed as it is, at half resolution, for
+// the real-pixel kernels (otherwise it is packed spread onto the stride-1 grid).
+WgradRowsJob wgrad_rows_prepare(const at::Tensor& input, int layout, int64_t Cout, at::Tensor& gw, at::Tensor* gb,
+                                int stride, bool px2) {
   WgradRowsJob j;
   j.B = input.size(0), j.Cin = input.size(1), j.H = input.size(2), j.W = input.size(3), j.Cout = Cout;
   j.layout = layout;
@@ -1078,7 +1120,10 @@ WgradRowsJob wgrad_rows_prepare(const at::Tensor& input, int layout, int64_t Cou
   } else {
     j.xpacked = pack_rows(input, layout);
   }
-  j.wsb = xdna_conv3x3_wgrad_rows_workspace_bytes(int(j.B), int(j.Cin), int(Cout), int(j.H), int(j.W), layout);
+  j.px = px2 ? 1 : stride == 1 && px_pick(kPxDw, input.sizes(), j.Cin, Cout, layout) ? 0 : -1;
+  j.wsb = j.px >= 0
+              ? xdna_conv3x3_px_wgrad_workspace_bytes(j.px, int(j.B), int(j.Cin), int(Cout), int(j.H), int(j.W))
+              : xdna_conv3x3_wgrad_rows_workspace_bytes(int(j.B), int(j.Cin), int(Cout), int(j.H), int(j.W), layout);
   j.ws = alloc_bytes(j.wsb);
   gw = empty_xdna({Cout, j.Cin, 3, 3}, at::kBFloat16);
   if (gb) *gb = empty_xdna({Cout}, at::kBFloat16);
@@ -1086,6 +1131,15 @@ WgradRowsJob wgrad_rows_prepare(const at::Tensor& input, int layout, int64_t Cou
 }
 
 void wgrad_rows_launch(const WgradRowsJob& j, const at::Tensor& dpacked, at::Tensor& gw, at::Tensor* gb, void* st) {
+  if (j.px >= 0) {
+    check_abi(xdna_conv3x3_px_wgrad_bf16(j.px, static_cast<const uint16_t*>(j.xpacked.const_data_ptr()),
+                                         static_cast<const uint16_t*>(dpacked.const_data_ptr()),
+                                         static_cast<uint16_t*>(gw.data_ptr()),
+                                         gb ? static_cast<uint16_t*>(gb->data_ptr()) : nullptr, int(j.B), int(j.Cin),
+                                         int(j.Cout), int(j.H), int(j.W), j.layout, j.ws.data_ptr(), j.wsb, st),
+              "conv wgrad pixels");
+    return;
+  }
   check_abi(xdna_conv3x3_wgrad_rows_bf16(static_cast<const uint16_t*>(j.xpacked.const_data_ptr()),
                                          static_cast<const uint16_t*>(dpacked.const_data_ptr()),
                                          static_cast<uint16_t*>(gw.data_ptr()),
@@ -1096,8 +1150,8 @@ void wgrad_rows_launch(const WgradRowsJob& j, const at::Tensor& dpacked, at::Ten
 }
 
 void hip_wgrad_rows(const at::Tensor& input, const at::Tensor& dpacked, int layout, int64_t Cout, at::Tensor& gw,
-                    at::Tensor* gb) {
-  const WgradRowsJob j = wgrad_rows_prepare(input, layout, Cout, gw, gb);
+                    at::Tensor* gb, int stride, bool px2) {
+  const WgradRowsJob j = wgrad_rows_prepare(input, layout, Cout, gw, gb, stride, px2);
   KernelTimer kt("conv3x3_wgrad", 2.0 * double(j.B) * double(j.H) * double(j.W) * double(j.Cin) * double(Cout) * 9.0);
   wgrad_rows_launch(j, dpacked, gw, gb, current_stream());
 }
@@ -1181,6 +1235,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
   const bool few_in = hip && !strided && few_input_3x3(input, weight);
   const bool dw = hip && mask[1] && g_mode.load() >= 2 && !few_in;
   const bool dw_rows = dw && wgrad_rows_pick(input.size(1), weight.size(0), input.size(3));
+  // a stride-2 conv on the real-pixel kernels: dY packed as it is, not spread
+  const bool px2 = strided && px_pick(kPxS2Dx, input.sizes(), weight.size(0), weight.size(1), g_conv_layout.load()) &&
+                   (!dw_rows || px_pick(kPxS2Dw, input.sizes(), input.size(1), weight.size(0), g_conv_layout.load()));
   // dY packed once: the input gradient's conv and the rows weight gradient read it
   const int layout = g_conv_layout.load();
   at::Tensor gop;
@@ -1188,7 +1245,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
   // the input gradient alone reads dY: a small grid reads it in place
   const bool dx_nchw = hip && mask[0] && !dx_few && !dw_rows && !strided && nchw_route(go, weight.size(1), true);
   if (hip && ((mask[0] && !dx_nchw && !dx_few) || dw_rows))
-    gop = strided ? pack_rows_spread(grad_output, go_sizes[2], go_sizes[3], layout) : pack_rows(go, layout);
+    gop = strided && !px2 ? pack_rows_spread(grad_output, go_sizes[2], go_sizes[3], layout) : pack_rows(go, layout);
   // the rows weight gradient beside the input gradient (captured graphs only)
   const bool both = dw_rows && mask[0];
   const int64_t ctag = both && g_wgrad_overlap.load() ? capture_tag() : 0;
@@ -1196,12 +1253,13 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
   const bool beside = ctag != 0 && side_stream_ready(false);
   WgradRowsJob wjob;
   if (beside) {
-    wjob = wgrad_rows_prepare(input, layout, weight.size(0), gw, mask[2] ? &gb : nullptr);
+    wjob = wgrad_rows_prepare(input, layout, weight.size(0), gw, mask[2] ? &gb : nullptr, strided ? 2 : 1, px2);
     check_abi(xdna_hip_event_record(g_side.fork, current_stream()), "conv backward fork");
   }
   if (hip && mask[0]) {
     ScopedCount sc("hip_conv3x3.dx.run");
     gi = dx_few    ? hip_gconv_dgrad(go, weight, gconv_geom(input, weight, stride, padding))
+         : px2     ? hip_conv_s2_dx(gop, layout, input.sizes(), weight)
          : dx_nchw ? hip_conv_nchw(go, weight, nullptr, true)
                    : hip_conv_packed(gop, layout, go_sizes, weight, nullptr, true, 0, !strided);
     mask[0] = false;
@@ -1226,7 +1284,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
         check_abi(xdna_hip_event_record(g_side.join, g_side.stream), "conv backward join");
         check_abi(xdna_hip_stream_wait_event(current_stream(), g_side.join), "conv backward join");
       } else {
-        hip_wgrad_rows(input, gop, layout, weight.size(0), gw, mask[2] ? &gb : nullptr);
+        hip_wgrad_rows(input, gop, layout, weight.size(0), gw, mask[2] ? &gb : nullptr, strided ? 2 : 1, px2);
       }
     } else {
       hip_wgrad(input, go, gw, mask[2] ? &gb : nullptr);

@@ -78,6 +78,10 @@ SIGNATURES = {
     "xdna_conv3x3_layout_rows_stride2_bf16": (I, [P, P, P, P, I, I, I, I, I, I, P]),
     "xdna_conv3x3_layout_pack_dilate2_bf16": (I, [P, P, I, I, I, I, I, P]),
     "xdna_conv3x3_layout_rows_bfp16_emul_bf16": (I, [P, P, P, P, I, I, I, I, I, I, I, P]),
+    "xdna_conv3x3_px_bf16": (I, [I, P, P, P, P] + [I] * 8 + [P]),
+    "xdna_conv3x3_px_pick": (I, [I] * 7),
+    "xdna_conv3x3_px_wgrad_workspace_bytes": (Z, [I] * 6),
+    "xdna_conv3x3_px_wgrad_bf16": (I, [I, P, P, P, P] + [I] * 6 + [P, Z, P]),
     "xdna_conv2d_fwd_bf16": (I, [P, P, P, P] + [I] * 11 + [P]),
     "xdna_instance_norm_fwd_bf16": (I, [P, P, P, I, P, P, P, L, L, L, ctypes.c_double, P]),
     "xdna_instance_norm_bwd_bf16": (I, [P, P, P, I, P, P, P, P, P, L, L, L, P]),
