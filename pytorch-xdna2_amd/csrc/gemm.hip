@@ -1406,13 +1406,14 @@ __device__ inline void sm_store(uint16_t* lds, const SmRegs& r, int64_t s_r, int
           make_uint4(r.u[4 * j], r.u[4 * j + 1], r.u[4 * j + 2], r.u[4 * j + 3]);
     }
   } else if (kMode == kAlongRow) {
+    // [64 k][8 pieces of 8 rows], piece q of k row kr at q ^ 4 ((kr >> 1) & 1): whole vectors,
+    // transposed by the fragment reads (four k rows x 64 bytes on 64 distinct banks)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int i = tid + j * 256;
-      const int kk = i >> 3, rv = (i & 7) * 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        lds[(rv + e) * kSmP + kk] = uint16_t((e & 1) ? (r.u[4 * j + (e >> 1)] >> 16) : (r.u[4 * j + (e >> 1)] & 0xFFFF));
+      const int kk = i >> 3, q = (i & 7) ^ (4 * ((i >> 4) & 1));
+      *reinterpret_cast<uint4*>(lds + kk * 64 + q * 8) =
+          make_uint4(r.u[4 * j], r.u[4 * j + 1], r.u[4 * j + 2], r.u[4 * j + 3]);
     }
   } else {
     const bool rows_fast = s_r == 1 && s_k != 1;
@@ -1425,47 +1426,86 @@ __device__ inline void sm_store(uint16_t* lds, const SmRegs& r, int64_t s_r, int
   }
 }
 
-template <int kModeA, int kModeB>
-__global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) uint16_t as[2][kSmT * kSmP];
-  __shared__ __attribute__((aligned(16))) uint16_t bs[2][kSmT * kSmP];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// MFMA fragment (rows rb + lane % 32, k = 16 ks + 8 (lane / 32) .. +7) of a staged k-tile.
+template <int kMode>
+__device__ inline u32x4_t sm_frag(const uint16_t* lds, int rb, int ks, int lane) {
+  if (kMode != kAlongRow) return *reinterpret_cast<const u32x4_t*>(lds + (rb + (lane & 31)) * kSmP + (lane >> 5) * 8 + ks * 16);
+  const int g = lane >> 4, j = lane & 15;
+  const int kr = 16 * ks + 8 * (g >> 1) + (j >> 2), r = rb + 16 * (g & 1) + 4 * (j & 3);
+  const uint16_t* p = lds + kr * 64 + (((r >> 3) ^ (4 * ((kr >> 1) & 1))) << 3) + (r & 7);
+  const g2u2 lo = __builtin_bit_cast(
+      g2u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) g4i16x4*)(p)));
+  const g2u2 hi = __builtin_bit_cast(
+      g2u2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) g4i16x4*)(p + 4 * 64)));
+  return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// G: thread groups of four waves, each multiplying its own share of the tile's k-tiles from LDS
+// buffers of its own; the groups' accumulators are added in order through LDS.  With 4 groups
+// a k of up to 16 k-tiles needs no second launch (see gemm_run).
+template <int kModeA, int kModeB, int G>
+__global__ __launch_bounds__(256 * G) void gemm_small_kernel(GemmArgs g) {
+  // (one group's buffers fit the static limit, and a kernel without dynamic LDS starts sooner)
+  extern __shared__ __attribute__((aligned(16))) uint16_t dyn[];
+  __shared__ __attribute__((aligned(16))) uint16_t fixed[G > 1 ? 1 : 4 * kSmT * kSmP];
+  uint16_t* smem = G > 1 ? dyn : fixed;
+  const int grp = G > 1 ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 8) : 0;
+  uint16_t* as = smem + grp * 4 * kSmT * kSmP;   // [2][kSmT * kSmP]
+  uint16_t* bs = as + 2 * kSmT * kSmP;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int m0 = blockIdx.y * kSmT, n0 = blockIdx.x * kSmT;
   const int batch = blockIdx.z / g.nsplit, split = blockIdx.z - batch * g.nsplit;
-  const int kbeg = split * g.kt_per * kSmK, kend = min(g.K, kbeg + g.kt_per * kSmK);
+  const int kt_grp = (g.kt_per + G - 1) / G;
+  const int kbeg = (split * g.kt_per + grp * kt_grp) * kSmK;
+  const int kend = min(min(g.K, (split + 1) * g.kt_per * kSmK), kbeg + kt_grp * kSmK);
   const uint16_t* A = g.a + int64_t(batch) * g.a_batch;
   const uint16_t* B = g.b + int64_t(batch) * g.b_batch;
-  const int lr = lane & 31, lk = (lane >> 5) * 8;
-
   f32x16_t acc = zero_acc();
   SmRegs ra, rb;
   if (kbeg < kend) {
     sm_load<kModeA>(ra, A, g.a_r, g.a_k, m0, g.M, kbeg, kend, tid);
     sm_load<kModeB>(rb, B, g.b_r, g.b_k, n0, g.N, kbeg, kend, tid);
-    sm_store<kModeA>(as[0], ra, g.a_r, g.a_k, tid);
-    sm_store<kModeB>(bs[0], rb, g.b_r, g.b_k, tid);
+    sm_store<kModeA>(as, ra, g.a_r, g.a_k, tid);
+    sm_store<kModeB>(bs, rb, g.b_r, g.b_k, tid);
   }
   __syncthreads();
   int buf = 0;
-  for (int k0 = kbeg; k0 < kend; k0 += kSmK) {
+  // every group runs the same number of rounds (a short one's are empty)
+  const int kstop = G > 1 ? kbeg + kt_grp * kSmK : kend;
+  for (int k0 = kbeg; k0 < kstop; k0 += kSmK) {
     const bool more = k0 + kSmK < kend;
     if (more) {  // the next k-tile's loads fly during this one's MFMAs
       sm_load<kModeA>(ra, A, g.a_r, g.a_k, m0, g.M, k0 + kSmK, kend, tid);
       sm_load<kModeB>(rb, B, g.b_r, g.b_k, n0, g.N, k0 + kSmK, kend, tid);
     }
-    const uint16_t* ab = as[buf] + (wm * 32 + lr) * kSmP + lk;
-    const uint16_t* bb = bs[buf] + (wn * 32 + lr) * kSmP + lk;
+    if (G == 1 || k0 < kend) {
+      const uint16_t* ab = as + buf * kSmT * kSmP;
+      const uint16_t* bb = bs + buf * kSmT * kSmP;
 #pragma unroll
-    for (int ks = 0; ks < kSmK / 16; ++ks)
-      acc = mfma_32x32x16(as_bf16x8(*reinterpret_cast<const uint4*>(ab + ks * 16)),
-                          as_bf16x8(*reinterpret_cast<const uint4*>(bb + ks * 16)), acc);
+      for (int ks = 0; ks < kSmK / 16; ++ks)
+        acc = mfma_32x32x16(as_bf16x8(sm_frag<kModeA>(ab, wm * 32, ks, lane)),
+                            as_bf16x8(sm_frag<kModeB>(bb, wn * 32, ks, lane)), acc);
+    }
     if (more) {  // the other buffer's last reads ended before the previous barrier
-      sm_store<kModeA>(as[buf ^ 1], ra, g.a_r, g.a_k, tid);
-      sm_store<kModeB>(bs[buf ^ 1], rb, g.b_r, g.b_k, tid);
+      sm_store<kModeA>(as + (buf ^ 1) * kSmT * kSmP, ra, g.a_r, g.a_k, tid);
+      sm_store<kModeB>(bs + (buf ^ 1) * kSmT * kSmP, rb, g.b_r, g.b_k, tid);
     }
     __syncthreads();
     buf ^= 1;
+  }
+  if (G > 1) {
+    float* red = reinterpret_cast<float*>(smem);  // [G - 1][16][256]
+    if (grp > 0) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[((grp - 1) * 16 + r) * 256 + tid] = acc[r];
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll
+    for (int q = 0; q < G - 1; ++q)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += red[(q * 16 + r) * 256 + tid];
   }
 
   // the tile, or (split-K) this split's fp32 partial tile
@@ -1473,11 +1513,40 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(GemmArgs g) {
   store_block<1, 1>(g, batch, split, out, m0 + wm * 32, n0 + wn * 32, lane);
 }
 
+constexpr size_t kSmLds = size_t(4) * kSmT * kSmP * 2;  // one group's buffers
+
+template <int MA, int MB>
+void launch_small(bool groups, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  if constexpr (MA != kScalar && MB != kScalar) {
+    if (groups) {
+      gemm_small_kernel<MA, MB, 4><<<grid, 1024, 4 * kSmLds, st>>>(g);
+      return;
+    }
+  }
+  gemm_small_kernel<MA, MB, 1><<<grid, 256, 0, st>>>(g);
+}
+
+// whether the four-group form's LDS can be had, for every operand form it takes
+bool small_groups_ok() {
+  static const bool ok = [] {
+    const auto set = [](const void* f) {
+      return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(4 * kSmLds)) == hipSuccess;
+    };
+    const bool r = set(reinterpret_cast<const void*>(&gemm_small_kernel<kAlongK, kAlongK, 4>)) &&
+                   set(reinterpret_cast<const void*>(&gemm_small_kernel<kAlongK, kAlongRow, 4>)) &&
+                   set(reinterpret_cast<const void*>(&gemm_small_kernel<kAlongRow, kAlongK, 4>)) &&
+                   set(reinterpret_cast<const void*>(&gemm_small_kernel<kAlongRow, kAlongRow, 4>));
+    if (!r) (void)hipGetLastError();
+    return r;
+  }();
+  return ok;
+}
+
 template <int MA>
-void launch_small_b(int mb, dim3 grid, hipStream_t st, const GemmArgs& g) {
-  if (mb == kAlongK) gemm_small_kernel<MA, kAlongK><<<grid, 256, 0, st>>>(g);
-  else if (mb == kAlongRow) gemm_small_kernel<MA, kAlongRow><<<grid, 256, 0, st>>>(g);
-  else gemm_small_kernel<MA, kScalar><<<grid, 256, 0, st>>>(g);
+void launch_small_b(int mb, bool groups, dim3 grid, hipStream_t st, const GemmArgs& g) {
+  if (mb == kAlongK) launch_small<MA, kAlongK>(groups, grid, st, g);
+  else if (mb == kAlongRow) launch_small<MA, kAlongRow>(groups, grid, st, g);
+  else launch_small<MA, kScalar>(groups, grid, st, g);
 }
 
 // Small products take gemm_small_kernel: a side of at most 128 or a k of at most 128, and
@@ -1614,8 +1683,13 @@ int gemm_run(const PartialsSource& src, const uint16_t* A, const uint16_t* Bm, u
     // per CU, each split keeping at least two k-tiles
     const int64_t tiles = ceil_div(M, kSmT) * ceil_div(N, kSmT) * int64_t(batch);
     const int ktiles = int(ceil_div(K, kSmK));
+    // few k-tiles: the four groups of a workgroup take them instead, and no partials or second
+    // launch are needed: up to 8 (128 x 1000 outputs, k 512: 6.7 us either way, one launch
+    // less for the host), up to 16 where the tiles alone fill a quarter of the chip (128 x 4096,
+    // k 1000: 13.9 -> 8.7; on 128 x 512 8.3 against 7.1)
+    const bool groups = tiles < 256 && ktiles >= 4 && ktiles <= (tiles >= 64 ? 16 : 8) && ma != kScalar && mb != kScalar && small_groups_ok();
     int nsplit = 1;
-    if (tiles < 256 && ktiles >= 4)
+    if (tiles < 256 && ktiles >= 4 && !groups)
       nsplit = int(std::max<int64_t>(1, std::min<int64_t>({ceil_div(512, tiles), int64_t(ktiles / 2),
                                                            int64_t(65535 / std::max(batch, 1))})));
     g.kt_per = int(ceil_div(ktiles, nsplit));
@@ -1627,9 +1701,9 @@ int gemm_run(const PartialsSource& src, const uint16_t* A, const uint16_t* Bm, u
     }
     const dim3 grid(unsigned(ceil_div(N, kSmT)), unsigned(ceil_div(M, kSmT)), unsigned(batch * g.nsplit));
     hipStream_t sts = as_stream(stream);
-    if (ma == kAlongK) launch_small_b<kAlongK>(mb, grid, sts, g);
-    else if (ma == kAlongRow) launch_small_b<kAlongRow>(mb, grid, sts, g);
-    else launch_small_b<kScalar>(mb, grid, sts, g);
+    if (ma == kAlongK) launch_small_b<kAlongK>(mb, groups, grid, sts, g);
+    else if (ma == kAlongRow) launch_small_b<kAlongRow>(mb, groups, grid, sts, g);
+    else launch_small_b<kScalar>(mb, groups, grid, sts, g);
     if (g.nsplit > 1) {
       launch_gemm_reduce(g, sts);
       src.give_back(g.part);  // stream-ordered reuse: the next user of the block runs after the reduce

@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 X = torch.device("xdna")
 
 
-@pytest.mark.parametrize("R,N", [(8192, 4096), (8192, 1024), (3, 5), (1, 7), (100, 8), (4096, 1002), (33, 4)])
+@pytest.mark.parametrize("R,N", [(8192, 4096), (8192, 1024), (3, 5), (1, 7), (100, 8), (4096, 1002), (33, 4),
+                                 (512, 36), (513, 36), (1, 4), (128, 1000), (31, 100)])
 def test_colsum_matches_fp64(hip, R, N):
     rng = np.random.default_rng(R * 7 + N)
     x = oracle.rng_bf16(rng, (R, N))

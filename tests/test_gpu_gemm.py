@@ -135,6 +135,23 @@ def test_mlp_shape(hip, variant):
     check_bf16(got, ref, what="mlp fwd")
 
 
+# k-tiles of 64: below and at the four-group form's limits (with few and with many tiles), a
+# last group without k-tiles or with part of one, a split K beyond; ragged rows and columns
+@pytest.mark.parametrize("M,N,K", [(128, 104, 512), (72, 64, 200), (8, 72, 264), (64, 64, 328), (40, 136, 520),
+                                   (128, 2056, 1000), (64, 4104, 1032), (24, 520, 2048)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_small_products(hip, M, N, K, layout):
+    """The small-product kernel in every vector layout, with a per-column bias, batched too."""
+    print(f"gemm small {layout} {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    a, b = oracle.rng_bf16(rng, (2, M, K)), oracle.rng_bf16(rng, (2, K, N))
+    ref = oracle.gemm(a, b)
+    da, a_s = (dev(a), (K, 1)) if layout[0] == "n" else (dev(np.ascontiguousarray(np.swapaxes(a, 1, 2))), (1, M))
+    db, b_s = (dev(b), (N, 1)) if layout[1] == "n" else (dev(np.ascontiguousarray(np.swapaxes(b, 1, 2))), (1, K))
+    check_bf16(_run(hip, da, db, M, N, K, a_s, b_s, batch=2, sa=M * K, sb=K * N), ref, what=f"{layout} batched")
+    check_bf16(_run(hip, da, db, M, N, K, a_s, b_s)[0], ref[0], what=layout)
+
+
 @pytest.mark.parametrize("bias_mode", [0, 2])
 def test_gram_split_k(hip, bias_mode):
     """Batched Gram products (few output tiles, long K): the split-K path, whose fp32
