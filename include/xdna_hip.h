@@ -662,6 +662,23 @@ int xdna_upsample_nearest2x_bwd_bf16(const uint16_t* dy, uint16_t* dx, int64_t p
 int xdna_subsample2_bf16(const uint16_t* full, uint16_t* y, int64_t planes, int H, int W, void* stream);
 int xdna_dilate2_bf16(const uint16_t* dy, uint16_t* full, int64_t planes, int H, int W, void* stream);
 
+/* 1x1 convs without padding, stride 1 or 2, read and written where they are: y[n][co][oy][ox]
+ * = the sum over ci of w[co][ci] x[n][ci][s oy][s ox] (+ bias, may be null), its input
+ * gradient (every dx element is written, zeros where the stride skips) and its weight
+ * gradient (fp32 partials in the workspace, added in a fixed order).  B x Cin x H x W input,
+ * ceil(H/s) x ceil(W/s) output planes; any 2-byte alignment, the workspace 4-byte aligned.
+ * The reference runs them on its CPU (torch_xdna_device.cpp:4524-4606, 4608-4885).
+ * xdna_conv1x1_pick(op, ...) is 1 where these are the faster form (op 0 forward, 1 input
+ * gradient, 2 weight gradient), 0 where the batched product of xdna_gemm_bf16 is. */
+int xdna_conv1x1_pick(int op, int B, int Cin, int Cout, int H, int W, int stride);
+int xdna_conv1x1_fwd_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int B, int Cin,
+                          int Cout, int H, int W, int stride, void* stream);
+int xdna_conv1x1_dgrad_bf16(const uint16_t* dy, const uint16_t* w, uint16_t* dx, int B, int Cin, int Cout, int H,
+                            int W, int stride, void* stream);
+size_t xdna_conv1x1_wgrad_workspace_bytes(int B, int Cin, int Cout, int H, int W, int stride);
+int xdna_conv1x1_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, int B, int Cin, int Cout, int H,
+                            int W, int stride, void* workspace, size_t workspace_bytes, void* stream);
+
 /* The same conv without the sampling passes (the backend's path for 3x3 / stride-2 /
  * pad-1 convs; the reference runs them on its CPU, torch_xdna_device.cpp:4524-4606,
  * 4608-4885):

@@ -929,11 +929,11 @@ at::Tensor hip_gconv_dgrad(const at::Tensor& grad, const at::Tensor& weight, con
 }
 
 // ---------------------------------------------------------------------------------------
-// 1x1 convolutions (stride 1 or 2, no padding: ResNet's downsampling shortcut) as MFMA
-// GEMMs: y[n] = W [Cout x Cin] . x[n] [Cin x HW] for every image (one batched launch with
-// the weight broadcast), dx[n] = W^T . dy[n], and dW = dY^T . X over all N*HW pixels as
-// one split-K product of channel-major copies.  Stride 2 takes every other pixel of x
-// (subsample2) and spreads dx back onto the full grid with zeros (dilate2).  The
+// 1x1 convolutions (stride 1 or 2, no padding: ResNet's downsampling shortcut): y[n] =
+// W [Cout x Cin] . x[n] [Cin x HW] for every image, dx[n] = W^T . dy[n], dW = dY^T . X over all
+// N*HW pixels.  The kernels of conv1x1.hip sample and spread in place; where xdna_conv1x1_pick
+// prefers the GEMM, the batched product has the weight broadcast, stride 2 samples x
+// (subsample2) and spreads dx back (dilate2), and dW is one product of channel-major copies.  The
 // reference runs these on its CPU (torch_xdna_device.cpp:4594-4604, 4862-4874).
 // ---------------------------------------------------------------------------------------
 bool conv1x1_eligible(const at::Tensor& x, const at::Tensor& w, c10::SymIntArrayRef stride,
@@ -964,7 +964,27 @@ at::Tensor conv1x1_input(const at::Tensor& input, int64_t s) {
   return xs;
 }
 
+// Whether the 1x1 kernels that sample and spread in place are the faster form (op 0 forward, 1
+// input gradient, 2 weight gradient); else the product runs on sampled or channel-major copies.
+bool conv1x1_direct(int op, const at::Tensor& x, int64_t Co, int64_t s) {
+  return xdna_conv1x1_pick(op, int(x.size(0)), int(x.size(1)), int(Co), int(x.size(2)), int(x.size(3)), int(s)) == 1;
+}
+
 at::Tensor hip_conv1x1_fwd(const at::Tensor& input, const at::Tensor& weight, const at::Tensor* bias, int64_t s) {
+  if (conv1x1_direct(0, input, weight.size(0), s)) {
+    const at::Tensor x = input.contiguous(), w = weight.contiguous();
+    const int64_t N = x.size(0), Ci = x.size(1), H = x.size(2), W = x.size(3), Co = w.size(0);
+    at::Tensor y = empty_xdna({N, Co, (H + s - 1) / s, (W + s - 1) / s}, at::kBFloat16), bc;
+    if (bias) bc = bias->contiguous();
+    KernelTimer kt("conv1x1.fwd", 2.0 * N * y.size(2) * y.size(3) * double(Co) * Ci);
+    check_abi(xdna_conv1x1_fwd_bf16(static_cast<const uint16_t*>(x.const_data_ptr()),
+                                    static_cast<const uint16_t*>(w.const_data_ptr()),
+                                    bias ? static_cast<const uint16_t*>(bc.const_data_ptr()) : nullptr,
+                                    static_cast<uint16_t*>(y.data_ptr()), int(N), int(Ci), int(Co), int(H), int(W),
+                                    int(s), current_stream()),
+              "conv1x1 forward");
+    return y;
+  }
   const at::Tensor xs = conv1x1_input(input, s);
   const at::Tensor w = weight.contiguous();
   const int64_t N = xs.size(0), Ci = xs.size(1), Ho = xs.size(2), Wo = xs.size(3), Co = w.size(0), P = Ho * Wo;
@@ -988,7 +1008,15 @@ void hip_conv1x1_bwd(const at::Tensor& grad_output, const at::Tensor& input, con
   const int64_t N = input.size(0), Ci = input.size(1), H = input.size(2), W = input.size(3);
   const int64_t Co = w.size(0), Ho = dy.size(2), Wo = dy.size(3), P = Ho * Wo;
   void* st = current_stream();
-  if (mask[0]) {
+  if (mask[0] && conv1x1_direct(1, input, Co, s)) {
+    gi = empty_xdna({N, Ci, H, W}, at::kBFloat16);
+    KernelTimer kt("conv1x1.dgrad", 2.0 * N * P * double(Co) * Ci);
+    check_abi(xdna_conv1x1_dgrad_bf16(static_cast<const uint16_t*>(dy.const_data_ptr()),
+                                      static_cast<const uint16_t*>(w.const_data_ptr()),
+                                      static_cast<uint16_t*>(gi.data_ptr()), int(N), int(Ci), int(Co), int(H), int(W),
+                                      int(s), st),
+              "conv1x1 input gradient");
+  } else if (mask[0]) {
     at::Tensor dxs = empty_xdna({N, Ci, Ho, Wo}, at::kBFloat16);
     KernelTimer kt("conv1x1.dgrad", 2.0 * N * P * double(Co) * Ci);
     check_abi(xdna_gemm_bf16(static_cast<const uint16_t*>(w.const_data_ptr()),
@@ -1005,7 +1033,19 @@ void hip_conv1x1_bwd(const at::Tensor& grad_output, const at::Tensor& input, con
                 "conv1x1 dilate");
     }
   }
-  if (mask[1]) {
+  if (mask[1] && conv1x1_direct(2, input, Co, s)) {
+    const at::Tensor x = input.contiguous();
+    const size_t wsb = xdna_conv1x1_wgrad_workspace_bytes(int(N), int(Ci), int(Co), int(H), int(W), int(s));
+    at::Tensor ws = alloc_bytes(wsb);
+    gw = empty_xdna({Co, Ci, 1, 1}, at::kBFloat16);
+    KernelTimer kt("conv1x1.wgrad", 2.0 * N * P * double(Co) * Ci);
+    check_abi(xdna_conv1x1_wgrad_bf16(static_cast<const uint16_t*>(x.const_data_ptr()),
+                                      static_cast<const uint16_t*>(dy.const_data_ptr()),
+                                      static_cast<uint16_t*>(gw.data_ptr()), int(N), int(Ci), int(Co), int(H), int(W),
+                                      int(s), ws.data_ptr(), wsb, st),
+              "conv1x1 weight gradient");
+    g_dw_jobs.fetch_add(1);
+  } else if (mask[1]) {
     // channel-major copies: dY^T [Co][N*P] and X^T [Ci][N*P], then one product over N*P
     const at::Tensor dyt = dy.permute({1, 0, 2, 3}).contiguous();
     const at::Tensor xst = conv1x1_input(input, s).permute({1, 0, 2, 3}).contiguous();

@@ -82,6 +82,11 @@ SIGNATURES = {
     "xdna_conv3x3_px_pick": (I, [I] * 7),
     "xdna_conv3x3_px_wgrad_workspace_bytes": (Z, [I] * 6),
     "xdna_conv3x3_px_wgrad_bf16": (I, [I, P, P, P, P] + [I] * 6 + [P, Z, P]),
+    "xdna_conv1x1_pick": (I, [I] * 7),
+    "xdna_conv1x1_fwd_bf16": (I, [P, P, P, P] + [I] * 6 + [P]),
+    "xdna_conv1x1_dgrad_bf16": (I, [P, P, P] + [I] * 6 + [P]),
+    "xdna_conv1x1_wgrad_workspace_bytes": (Z, [I] * 6),
+    "xdna_conv1x1_wgrad_bf16": (I, [P, P, P] + [I] * 6 + [P, Z, P]),
     "xdna_conv2d_fwd_bf16": (I, [P, P, P, P] + [I] * 11 + [P]),
     "xdna_instance_norm_fwd_bf16": (I, [P, P, P, I, P, P, P, L, L, L, ctypes.c_double, P]),
     "xdna_instance_norm_bwd_bf16": (I, [P, P, P, I, P, P, P, P, P, L, L, L, P]),
