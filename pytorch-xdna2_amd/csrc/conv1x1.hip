@@ -29,10 +29,6 @@
 namespace xdna {
 namespace {
 
-struct __attribute__((packed, aligned(2))) Pix8 {
-  uint32_t v[4];
-};
-
 struct __attribute__((packed, aligned(2))) Pix2 {
   uint32_t v;
 };

@@ -35,10 +35,6 @@ constexpr int kFewThreads = 512;          // weight gradient: its staging is lat
 constexpr int kFewWeights = 16;           // weight loads in flight per thread
 
 // Eight pixels of one channel at any 2-byte address.
-struct __attribute__((packed, aligned(2))) Pix8 {
-  uint32_t v[4];
-};
-
 // Every kernel below may use up to a CU's LDS.
 bool raise_lds(const void* fn) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(kFewLdsMax)) == hipSuccess;

@@ -40,9 +40,8 @@ __device__ inline float go_value(const void* go, int go_dtype) {
 
 // Row-major index (0..3) of the window maximum: (0,0), (0,1), (1,0), (1,1); a value
 // replaces the running maximum when it is larger or NaN (PyTorch's max_pool2d rule).
-__device__ inline int window_argmax(const uint16_t* w0, int W, float& m) {
-  const float v[4] = {bf16_to_f32(w0[0]), bf16_to_f32(w0[1]), bf16_to_f32(w0[W]), bf16_to_f32(w0[W + 1])};
-  m = -INFINITY;
+__device__ inline int argmax4(const float (&v)[4], float* max = nullptr) {
+  float m = -INFINITY;
   int k = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -50,6 +49,7 @@ __device__ inline int window_argmax(const uint16_t* w0, int W, float& m) {
       m = v[j];
       k = j;
     }
+  if (max) *max = m;
   return k;
 }
 
@@ -62,8 +62,10 @@ __global__ __launch_bounds__(kRegionThreads) void maxpool2_kernel(const uint16_t
     const int64_t p = i / (int64_t(Ho) * Wo);
     const int r = int(i - p * Ho * Wo);
     const int oy = r / Wo, ox = r - oy * Wo;
+    const uint16_t* w0 = x + (p * H + 2 * oy) * W + 2 * ox;
+    const float v[4] = {bf16_to_f32(w0[0]), bf16_to_f32(w0[1]), bf16_to_f32(w0[W]), bf16_to_f32(w0[W + 1])};
     float m;
-    window_argmax(x + (p * H + 2 * oy) * W + 2 * ox, W, m);
+    argmax4(v, &m);
     y[i] = f32_to_bf16(m);
   }
 }
@@ -84,56 +86,123 @@ struct BwdArgs {
   int H, W, Ho, Wo;
 };
 
-__global__ __launch_bounds__(kRegionThreads) void region_bwd_kernel(BwdArgs a) {
-  const int64_t n = a.planes * a.H * a.W;
-  const float s = a.ta ? a.scale * go_value(a.go, a.go_dtype) : 0.0f;
-  for (int64_t i = int64_t(blockIdx.x) * kRegionThreads + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * kRegionThreads) {
-    if (a.r && bf16_to_f32(a.r[i]) <= 0.0f) {
-      a.out[i] = 0;
-      continue;
-    }
-    float v = 0.0f;
-    if (a.g) {
-      v = bf16_to_f32(a.g[i]);
-    } else if (a.gp) {
-      const int64_t p = i / (int64_t(a.H) * a.W);
-      const int rem = int(i - p * a.H * a.W);
-      const int y = rem / a.W, x = rem - y * a.W;
-      const int oy = y >> 1, ox = x >> 1;
-      if (oy < a.Ho && ox < a.Wo) {
-        float m;
-        const int k = window_argmax(a.px + (p * a.H + 2 * oy) * a.W + 2 * ox, a.W, m);
-        if (k == ((y & 1) << 1) + (x & 1)) v = bf16_to_f32(a.gp[(p * a.Ho + oy) * a.Wo + ox]);
-      }
-    }
-    if (a.extra) v += bf16_to_f32(a.extra[i]);
-    if (a.ta) v += s * (bf16_to_f32(a.ta[i]) - bf16_to_f32(a.tb[i]));
-    a.out[i] = f32_to_bf16(v);
+// Four values from p, of which n are in the tensor (the others are 0).
+struct Vals4 {
+  float v[4];
+};
+
+__device__ inline Vals4 load4(const uint16_t* p, int n) {
+  Vals4 o = {{0.0f, 0.0f, 0.0f, 0.0f}};
+  if (n >= 4) {
+    const Pix4 a = *reinterpret_cast<const Pix4*>(p);
+    o.v[0] = bf16_to_f32(uint16_t(a.lo)), o.v[1] = bf16_to_f32(uint16_t(a.lo >> 16));
+    o.v[2] = bf16_to_f32(uint16_t(a.hi)), o.v[3] = bf16_to_f32(uint16_t(a.hi >> 16));
+  } else {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      if (u < n) o.v[u] = bf16_to_f32(p[u]);
+  }
+  return o;
+}
+
+__device__ inline void store4(uint16_t* p, int n, const float (&v)[4]) {
+  uint16_t h[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) h[u] = f32_to_bf16(v[u]);
+  if (n >= 4) {
+    *reinterpret_cast<Pix4*>(p) = Pix4{h[0] | (uint32_t(h[1]) << 16), h[2] | (uint32_t(h[3]) << 16)};
+  } else {
+#pragma unroll
+    for (int u = 0; u < 3; ++u)
+      if (u < n) p[u] = h[u];
   }
 }
 
-// part[blockIdx.x] = scale * sum over this block's elements of d^2, d = a - b (kind 0, both
-// bf16) or d = a / chw - t (kind 1: a the bf16 Gram matrices [batch][cc], t fp32 targets
-// with batch stride t_bstride, 0 for one target broadcast over the batch).  Block b sums
-// elements b * 256 + tid + k * gridDim.x * 256 in that order per thread, then a fixed tree.
-__global__ __launch_bounds__(kRegionThreads) void sqdiff_kernel(int kind, const uint16_t* __restrict__ a,
-                                                                const uint16_t* __restrict__ b,
-                                                                const float* __restrict__ t, int64_t t_bstride,
-                                                                int64_t cc, float chw, int64_t n, float scale,
-                                                                float* __restrict__ part) {
-  float s = 0.0f;
-  for (int64_t i = int64_t(blockIdx.x) * kRegionThreads + threadIdx.x; i < n;
-       i += int64_t(gridDim.x) * kRegionThreads) {
-    float d;
-    if (kind == 0) {
-      d = bf16_to_f32(a[i]) - bf16_to_f32(b[i]);
-    } else {
-      const int64_t bi = i / cc;
-      d = bf16_to_f32(a[i]) / chw - t[bi * t_bstride + (i - bi * cc)];
-    }
-    s = fmaf(d, d, s);
+// The mask and the terms beside the base gradient of n elements from i.
+__device__ inline void region_terms(const BwdArgs& a, float s, int64_t i, int n, float (&v)[4]) {
+  if (a.extra) {
+    const Vals4 e = load4(a.extra + i, n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] += e.v[u];
   }
+  if (a.ta) {
+    const Vals4 x = load4(a.ta + i, n), y = load4(a.tb + i, n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] += s * (x.v[u] - y.v[u]);
+  }
+  if (a.r) {
+    const Vals4 r = load4(a.r + i, n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = r.v[u] <= 0.0f ? 0.0f : v[u];
+  }
+}
+
+// Memory bound: four elements per thread, the loads of all terms in flight before the mask is
+// known (one element per thread, masked before its other loads, was a chain of two or three
+// latencies on 2-byte loads; us on 40 x 64 x 36 x 36, a tensor 1.3: r and g 9.7 -> 4.6, with
+// extra and a tap 10.3 -> 5.7).
+__global__ __launch_bounds__(kRegionThreads) void region_bwd_kernel(BwdArgs a) {
+  const int64_t n = a.planes * a.H * a.W;
+  const float s = a.ta ? a.scale * go_value(a.go, a.go_dtype) : 0.0f;
+  for (int64_t i = (int64_t(blockIdx.x) * kRegionThreads + threadIdx.x) * 4; i < n;
+       i += int64_t(gridDim.x) * kRegionThreads * 4) {
+    const int m = int(std::min<int64_t>(4, n - i));
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (a.g) {
+      const Vals4 g = load4(a.g + i, m);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = g.v[u];
+    }
+    region_terms(a, s, i, m, v);
+    store4(a.out + i, m, v);
+  }
+}
+
+// Through the max-pool: a thread takes four columns of the two rows of a window row, so a
+// window's maximum is found once, not by each of its pixels (40 x 64 x 36 x 36 with extra: 14.4
+// -> 6.2 us).  I: the index type that holds the item count.
+template <class I>
+__global__ __launch_bounds__(kRegionThreads) void region_bwd_pool_kernel(BwdArgs a) {
+  const I wq = I((a.W + 3) / 4), hq = I((a.H + 1) / 2), n = I(a.planes) * hq * wq;
+  const float s = a.ta ? a.scale * go_value(a.go, a.go_dtype) : 0.0f;
+  for (I i = I(blockIdx.x) * kRegionThreads + threadIdx.x; i < n; i += I(gridDim.x) * kRegionThreads) {
+    const I row = i / wq;
+    const int x = 4 * int(i - row * wq);
+    const I p = row / hq;
+    const int oy = int(row - p * hq), y = 2 * oy, m = min(4, a.W - x);
+    const int64_t at = (int64_t(p) * a.H + y) * a.W + x;
+    const bool two = y + 1 < a.H;
+    float v[2][4] = {};
+    if (two) {
+      const Vals4 r0 = load4(a.px + at, m), r1 = load4(a.px + at + a.W, m);
+      const uint16_t* gp = a.gp + (int64_t(p) * a.Ho + oy) * a.Wo + (x >> 1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (2 * j + 1 >= m) continue;  // no window (an odd last column)
+        const float w[4] = {r0.v[2 * j], r0.v[2 * j + 1], r1.v[2 * j], r1.v[2 * j + 1]};
+        const float g = bf16_to_f32(gp[j]);
+        const int k = argmax4(w);
+        v[0][2 * j] = k == 0 ? g : 0.0f;
+        v[0][2 * j + 1] = k == 1 ? g : 0.0f;
+        v[1][2 * j] = k == 2 ? g : 0.0f;
+        v[1][2 * j + 1] = k == 3 ? g : 0.0f;
+      }
+    }
+    region_terms(a, s, at, m, v[0]);
+    store4(a.out + at, m, v[0]);
+    if (two) {
+      region_terms(a, s, at + a.W, m, v[1]);
+      store4(a.out + at + a.W, m, v[1]);
+    }
+  }
+}
+
+struct __attribute__((packed, aligned(4))) F32x4 {
+  float v[4];
+};
+
+// part[blockIdx.x] = scale * the block's sum of s, by a fixed tree
+__device__ inline void block_part(float s, float scale, float* part) {
   __shared__ float red[kRegionThreads];
   red[threadIdx.x] = s;
   __syncthreads();
@@ -142,6 +211,55 @@ __global__ __launch_bounds__(kRegionThreads) void sqdiff_kernel(int kind, const 
     __syncthreads();
   }
   if (threadIdx.x == 0) part[blockIdx.x] = scale * red[0];
+}
+
+// part[blockIdx.x] = scale * sum over this block's elements of (a - b)^2.  Block b sums
+// elements b * 256 + tid + k * gridDim.x * 256 in that order per thread, then a fixed tree.
+// (Wider runs per thread leave half of the blocks without work at 3.3M elements: 3.8 us so,
+// 4.4 with eight.)
+__global__ __launch_bounds__(kRegionThreads) void sqdiff_kernel(const uint16_t* __restrict__ a,
+                                                                const uint16_t* __restrict__ b, int64_t n,
+                                                                float scale, float* __restrict__ part) {
+  float s = 0.0f;
+  for (int64_t i = int64_t(blockIdx.x) * kRegionThreads + threadIdx.x; i < n;
+       i += int64_t(gridDim.x) * kRegionThreads) {
+    const float d = bf16_to_f32(a[i]) - bf16_to_f32(b[i]);
+    s = fmaf(d, d, s);
+  }
+  block_part(s, scale, part);
+}
+
+// The same of (G / chw - t)^2: G the bf16 Gram matrices [batch][cc], t fp32 targets with batch
+// stride t_bstride, 0 for one target broadcast over the batch.  A thread sums runs of eight (at
+// 8 (b * 256 + tid) + k * gridDim.x * 2048) in order; a run lies in one matrix where cc % 8 == 0,
+// so its index is divided once, in 32 bits where it fits (a 64-bit division per element held
+// 40 matrices of 512 x 512 to 14.2 us; now 8.0, the bytes' time is 4).
+__global__ __launch_bounds__(kRegionThreads) void gram_sqdiff_kernel(const uint16_t* __restrict__ G,
+                                                                     const float* __restrict__ t, int64_t t_bstride,
+                                                                     int64_t cc, float chw, int64_t n, float scale,
+                                                                     float* __restrict__ part) {
+  float s = 0.0f;
+  for (int64_t i = (int64_t(blockIdx.x) * kRegionThreads + threadIdx.x) * 8; i < n;
+       i += int64_t(gridDim.x) * kRegionThreads * 8) {
+    if (i + 8 <= n && cc % 8 == 0) {
+      const Pix8 x = *reinterpret_cast<const Pix8*>(G + i);
+      const int64_t bi = (i | cc) >> 32 ? i / cc : uint32_t(i) / uint32_t(cc);
+      const float* tp = t + bi * t_bstride + (i - bi * cc);
+      const F32x4 lo = *reinterpret_cast<const F32x4*>(tp), hi = *reinterpret_cast<const F32x4*>(tp + 4);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float d = bf16_to_f32(uint16_t(x.v[u >> 1] >> (16 * (u & 1)))) / chw - (u < 4 ? lo.v[u & 3] : hi.v[u & 3]);
+        s = fmaf(d, d, s);
+      }
+    } else {
+      for (int64_t e = i; e < i + 8 && e < n; ++e) {
+        const int64_t bi = e / cc;
+        const float d = bf16_to_f32(G[e]) / chw - t[bi * t_bstride + (e - bi * cc)];
+        s = fmaf(d, d, s);
+      }
+    }
+  }
+  block_part(s, scale, part);
 }
 
 // loss = sum of part[0 .. n) in fp64, thread-strided then a fixed tree; written as fp32
@@ -169,35 +287,59 @@ __global__ __launch_bounds__(kFinishThreads) void finish_kernel(const float* __r
 // S = bf16(coef * go * (d_ij + d_ji) / chw), d = G / chw - t, over C x C matrices: with
 // G = F F^T, the gradient of coef / 2 * sum d^2 with respect to F is S F (both operands of
 // the Gram product carry F), so one product gives it (coef = 2 w / N for w times a mean).
-// Block (tj, ti, b) takes the 32 x 32 tile at rows ti*32, columns tj*32 of matrix b and
-// stages the mirrored tile (rows tj*32, columns ti*32) of d in LDS, so both reads and the
-// write are coalesced.
+// S is symmetric, so a block takes the 32 x 32 tile at (ti, tj) of matrix blockIdx.z and
+// its mirror image: d is read once, four elements per thread, exchanged through LDS, and
+// both tiles are written.  The grid folds tile row y onto row nt - 1 - y: nt + 1 tiles on or
+// above the diagonal per pair of rows (x first the row's, then its partner's).  40 matrices of
+// 512 x 512: 25.2 us with every tile and its mirror read by its own block -> 13.9 (bytes: 8).
 constexpr int kGT = 32;
 
 __global__ __launch_bounds__(kRegionThreads) void gram_grad_kernel(const uint16_t* __restrict__ G,
                                                                    const float* __restrict__ t, int64_t t_bstride,
                                                                    int C, float chw, float coef, const void* go,
                                                                    int go_dtype, uint16_t* __restrict__ S) {
+  const int nt = (C + kGT - 1) / kGT;
+  int ti = blockIdx.y, tj = ti + int(blockIdx.x);
+  if (tj >= nt) {
+    if (nt - 1 - ti == ti) return;  // the middle row has no partner
+    tj = int(blockIdx.x) - (nt - ti);
+    ti = nt - 1 - ti;
+    tj += ti;
+  }
   const float c = coef * go_value(go, go_dtype);
   const int64_t cc = int64_t(C) * C;
-  const int b = blockIdx.z, i0 = blockIdx.y * kGT, j0 = blockIdx.x * kGT;
-  const uint16_t* Gb = G + b * cc;
-  const float* tb = t + b * t_bstride;
-  __shared__ float mir[kGT][kGT + 1];  // mir[x][y] = d at row j0 + y, column i0 + x
-  const int tx = threadIdx.x % kGT, ty = threadIdx.x / kGT;  // 32 x 8
-  for (int y = ty; y < kGT; y += kRegionThreads / kGT) {
-    const int r = j0 + y, col = i0 + tx;
-    float d = 0.0f;
-    if (r < C && col < C) d = bf16_to_f32(Gb[int64_t(r) * C + col]) / chw - tb[int64_t(r) * C + col];
-    mir[tx][y] = d;
+  const uint16_t* Gb = G + blockIdx.z * cc;
+  const float* tb = t + blockIdx.z * t_bstride;
+  uint16_t* Sb = S + blockIdx.z * cc;
+  __shared__ float tile[2][kGT][kGT + 1];
+  const int y = threadIdx.x / 8, x = 4 * (threadIdx.x % 8);
+  float d[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {  // the tile, its mirror
+    const int r = (h ? tj : ti) * kGT + y, col = (h ? ti : tj) * kGT + x;
+    const int64_t e = int64_t(r) * C + col;
+    const int m = r < C ? C - col : 0;
+    const Vals4 g = load4(Gb + e, m);
+    F32x4 w = {{0.0f, 0.0f, 0.0f, 0.0f}};
+    if (m >= 4) {
+      w = *reinterpret_cast<const F32x4*>(tb + e);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 3; ++u)
+        if (u < m) w.v[u] = tb[e + u];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) tile[h][y][x + u] = d[h][u] = g.v[u] / chw - w.v[u];
   }
   __syncthreads();
-  for (int y = ty; y < kGT; y += kRegionThreads / kGT) {
-    const int r = i0 + y, col = j0 + tx;
-    if (r >= C || col >= C) continue;
-    const int64_t e = int64_t(r) * C + col;
-    const float d = bf16_to_f32(Gb[e]) / chw - tb[e];
-    S[b * cc + e] = f32_to_bf16(c * (d + mir[y][tx]) / chw);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    if (h && ti == tj) break;
+    const int r = (h ? tj : ti) * kGT + y, col = (h ? ti : tj) * kGT + x;
+    float v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = c * (d[h][u] + tile[h ^ 1][x + u][y]) / chw;
+    store4(Sb + int64_t(r) * C + col, r < C ? C - col : 0, v);
   }
 }
 
@@ -243,7 +385,15 @@ int xdna_region_backward_bf16(const uint16_t* r, const uint16_t* g, const uint16
   }
   if (!admit_launch("xdna_region_backward_bf16")) return -1;
   BwdArgs a{r, g, gp, px, extra, ta, tb, go, go_dtype, scale, out, planes, H, W, H / 2, W / 2};
-  region_bwd_kernel<<<grid_for(n), kRegionThreads, 0, as_stream(stream)>>>(a);
+  if (!g && gp) {
+    const int64_t items = planes * ceil_div(H, 2) * ceil_div(W, 4);
+    if (items < (int64_t(1) << 31))
+      region_bwd_pool_kernel<uint32_t><<<grid_for(items), kRegionThreads, 0, as_stream(stream)>>>(a);
+    else
+      region_bwd_pool_kernel<int64_t><<<grid_for(items), kRegionThreads, 0, as_stream(stream)>>>(a);
+  } else {
+    region_bwd_kernel<<<grid_for(ceil_div(n, 4)), kRegionThreads, 0, as_stream(stream)>>>(a);
+  }
   return check_launch("xdna_region_backward_bf16");
 }
 
@@ -256,8 +406,7 @@ int xdna_region_sqdiff_bf16(const uint16_t* a, const uint16_t* b, int64_t n, flo
     return -1;
   }
   if (!admit_launch("xdna_region_sqdiff_bf16")) return -1;
-  sqdiff_kernel<<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(0, a, b, nullptr, 0, 1, 1.0f, n, scale,
-                                                                     part);
+  sqdiff_kernel<<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(a, b, n, scale, part);
   return check_launch("xdna_region_sqdiff_bf16");
 }
 
@@ -268,8 +417,8 @@ int xdna_region_gram_sqdiff_bf16(const uint16_t* G, const float* t, int64_t t_bs
     return -1;
   }
   if (!admit_launch("xdna_region_gram_sqdiff_bf16")) return -1;
-  sqdiff_kernel<<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(1, G, nullptr, t, t_bstride, cc, chw,
-                                                                     batch * cc, scale, part);
+  gram_sqdiff_kernel<<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(G, t, t_bstride, cc, chw, batch * cc,
+                                                                          scale, part);
   return check_launch("xdna_region_gram_sqdiff_bf16");
 }
 
@@ -297,7 +446,7 @@ int xdna_region_gram_grad_bf16(const uint16_t* G, const float* t, int64_t t_bstr
   }
   if (!admit_launch("xdna_region_gram_grad_bf16")) return -1;
   const unsigned nt = unsigned(ceil_div(C, kGT));
-  gram_grad_kernel<<<dim3(nt, nt, unsigned(batch)), kRegionThreads, 0, as_stream(stream)>>>(G, t, t_bstride, C, chw,
+  gram_grad_kernel<<<dim3(nt + 1, (nt + 1) / 2, unsigned(batch)), kRegionThreads, 0, as_stream(stream)>>>(G, t, t_bstride, C, chw,
                                                                                         coef, go, go_dtype, S);
   return check_launch("xdna_region_gram_grad_bf16");
 }

@@ -346,3 +346,64 @@ def test_region_step_captured_and_replayed():
         assert torch.equal(gl.detach().cpu(), eager_loss)
         assert torch.equal(x.grad.cpu(), eager_grad)
     gr.reset()
+
+
+# Vector forms of the loss and backward kernels at their edges: runs of four and eight with every
+# remainder, operands 2 bytes off a 4-byte address, planes of odd sizes (pixels without a window),
+# one row or column, Gram matrices of an odd, an even and one number of 32 x 32 tiles.
+@pytest.mark.parametrize("shape,off", [((2, 3, 7, 9), 1), ((1, 2, 5, 6), 0), ((3, 1, 2, 3), 1), ((1, 4, 1, 8), 0),
+                                       ((2, 2, 9, 1), 0), ((1, 1, 4, 11), 1), ((1, 1, 64, 37), 0)])
+def test_backward_pass_edges(shape, off):
+    g = torch.Generator().manual_seed(31 + sum(shape))
+
+    def at_off(t):  # contiguous, `off` elements into its storage
+        buf = torch.zeros(t.numel() + off, dtype=t.dtype).to(X)
+        buf[off:].copy_(t.reshape(-1).to(X))
+        return buf[off:].view(t.shape)
+
+    x = torch.randn(shape, generator=g).bfloat16()
+    x = torch.where(torch.rand(shape, generator=g) < 0.3, torch.zeros(()).bfloat16(), x)  # ties
+    gp = torch.randn(shape[0], shape[1], shape[2] // 2, shape[3] // 2, generator=g).bfloat16()
+    ex, ta, tb, gg = (torch.randn(shape, generator=g).bfloat16() for _ in range(4))
+    rr = torch.relu(x).float().requires_grad_()
+    routed = torch.zeros(shape)
+    if gp.numel():
+        torch.nn.functional.max_pool2d(rr, 2, 2).backward(gp.float())
+        routed = rr.grad
+    for base, kw in ((routed, (None, at_off(gp), at_off(torch.relu(x)))), (gg.float(), (at_off(gg), None, None))):
+        out = C().region_backward(at_off(torch.relu(x)), *kw, at_off(ex), at_off(ta), at_off(tb), 0.5, None, list(shape))
+        v = base.double() + ex.double() + 0.5 * (ta.double() - tb.double())
+        ref = torch.where(x.double() > 0, v, torch.zeros((), dtype=torch.float64))
+        # one rounding of an fp32 sum of terms below 16: half a bf16 ulp and three fp32 ulps of 16
+        assert ((out.cpu().double() - ref).abs() <= ref.abs() * 2.0 ** -8 + 3 * 2.0 ** -20).all()
+        out = C().region_backward(None, *kw, None, None, None, 0.0, None, list(shape))
+        np.testing.assert_array_equal(bits(out), bits(base.bfloat16()))
+
+
+@pytest.mark.parametrize("B,n,per_batch,off", [(3, 1, False, 0), (2, 31, True, 1), (1, 32, False, 0), (2, 66, True, 0),
+                                               (1, 97, True, 1), (2, 128, True, 0)])
+def test_gram_term_edges(B, n, per_batch, off):
+    g = torch.Generator().manual_seed(n)
+
+    def at_off(t):
+        buf = torch.zeros(t.numel() + off, dtype=t.dtype).to(X)
+        buf[off:].copy_(t.reshape(-1).to(X))
+        return buf[off:].view(t.shape)
+
+    G = (torch.randn(B, n, n, generator=g) * 50).bfloat16()
+    T = torch.randn(B if per_batch else 1, n, n, generator=g)
+    chw = 37.0 * n
+    d = G.double() / chw - T.double()
+    S = C().region_gram_grad(at_off(G), at_off(T), chw, 0.01, None)
+    ref = 0.01 * (d + d.transpose(1, 2)) / chw
+    # one bf16 rounding, and d's fp32 error where d_ij + d_ji cancels
+    tol = ref.abs() * 2.0 ** -8 + 2.0 ** -21 * 0.01 * (d.abs() + d.abs().transpose(1, 2)) / chw
+    assert ((S.cpu().double() - ref).abs() <= tol + 1e-30).all()
+    P = C().region_loss_parts()
+    part = torch.empty(2 * P, dtype=torch.float32, device=X)
+    C().region_gram_sqdiff(at_off(G), at_off(T), chw, 3.0, part, 0)
+    a, b = torch.randn(B * n * n, generator=g).bfloat16(), torch.randn(B * n * n, generator=g).bfloat16()
+    C().region_sqdiff(at_off(a), at_off(b), 0.25, part, P)
+    got = part.cpu().double().view(2, P).sum(1)
+    ref = torch.stack((3.0 * (d ** 2).sum(), 0.25 * ((a.double() - b.double()) ** 2).sum()))
+    assert ((got - ref).abs() <= 1e-5 * ref).all()
