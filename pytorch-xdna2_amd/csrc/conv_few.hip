@@ -34,7 +34,6 @@ constexpr size_t kFewLdsMax = 156 * 1024;  // a CU's 160 KiB less the block redu
 constexpr int kFewThreads = 512;          // weight gradient: its staging is latency, so more loads per workgroup
 constexpr int kFewWeights = 16;           // weight loads in flight per thread
 
-// Eight pixels of one channel at any 2-byte address.
 // Every kernel below may use up to a CU's LDS.
 bool raise_lds(const void* fn) {
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(kFewLdsMax)) == hipSuccess;
@@ -708,7 +707,8 @@ int conv_few_wgrad(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t
   a.Wf = few_dy ? a.Wo : W;
   a.KH = KH; a.KW = KW; a.ph = ph; a.pw = pw;
   a.M = a.Cf * KW;
-  if (a.Cf > 4 || a.Cw < 8 || KH > 8 * kFewMaxKy || KW < 3 || a.M > 32 || a.Ww < 4) return 1;
+  // (pw <= KW: a shifted row then stays within the zeros kept around it)
+  if (pw > KW || a.Cf > 4 || a.Cw < 8 || KH > 8 * kFewMaxKy || KW < 3 || a.M > 32 || a.Ww < 4) return 1;
   a.Wq = (a.Ww + 7) & ~7;
   a.wblks = int(ceil_div(a.Cw, 32));
   const int64_t total = int64_t(a.wblks) * KH * a.M * 32 + Cout;

@@ -110,6 +110,8 @@ FEW = [
     (2, 3, 70, 13, 17, 9, 9, 1, 1, 4, 4), (3, 1, 40, 7, 9, 5, 3, 1, 1, 0, 0), (2, 4, 33, 12, 20, 3, 5, 1, 1, 2, 4),
     (1, 2, 9, 6, 130, 7, 7, 1, 1, 3, 3), (1, 40, 3, 6, 150, 9, 9, 1, 1, 4, 4), (2, 32, 3, 16, 10, 1, 9, 1, 1, 0, 8),
     (5, 3, 64, 20, 27, 3, 3, 1, 1, 1, 1), (2, 9, 2, 11, 12, 16, 9, 1, 1, 8, 4), (700, 3, 16, 4, 4, 3, 3, 1, 1, 1, 1),
+    # paddings up to a kernel's width and past it
+    (2, 16, 3, 7, 9, 3, 3, 1, 1, 3, 3), (2, 3, 16, 7, 9, 3, 3, 1, 1, 6, 7), (2, 16, 3, 7, 9, 3, 3, 1, 1, 5, 6),
 ]
 
 
