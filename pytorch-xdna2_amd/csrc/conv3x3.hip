@@ -3526,8 +3526,7 @@ int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int lay
   if (op >= 3 && (g_wgrad_rows_form.load() != 0 || g_wgrad_tile.load() != 0)) return 0;
   const int form = op == 0 || op == 3 ? kPxStride1 : op == 2 ? kPxS2Dgrad : kPxStride2;
   if (op < 0 || op > 4 || !conv_px_fits(form, B, cin, cout, H, W, layout)) return 0;
-  // (the weight gradient reads dY's packed rows, too)
-  if (op >= 3 && !conv_px_fits(kPxStride1, B, cout, cin, H, W, layout)) return 0;
+  if (op >= 3 && !conv_px_wgrad_fits(form, B, cin, cout, H, W, layout)) return 0;
   if (op == 1 || op == 2 || op == 4) return 1;
   if (op == 0) {
     // grids the window kernels leave to their small-grid form, from 256 input channels: 256ch
@@ -3537,16 +3536,23 @@ int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int lay
     const ConvGeom g = conv_geom(B, H, W, layout);
     return cin > 3 * kKStep && ceil_div(g.m_total, 256) * ceil_div(cout, kSCo) < 150;
   }
-  // the weight gradient: up to 30 GFLOP (128ch 40 x 36 x 36 36.4 -> 29.9 us, 40 x 9 x 9 20.2 ->
-  // 15.9, 512ch 16 x 18 x 18 52.9 -> 45.0; beyond, 128ch 128 x 32 x 32 60.6 against 63), on one
-  // chunk of input channels (64ch 128 x 64 x 64 64.2 -> 57.1) and on images whose padded grid
-  // is half border (512ch 128 x 8 x 8 69.5 -> 56.7)
-  const double gflop = 2.0 * 9.0 * double(B) * H * W * double(cin) * double(cout) * 1e-9;
-  return cin <= kKStep || gflop <= 30.0 || H * W <= 64;
+  // the weight gradient, on `border` packed rows per pixel: the window kernels have the higher
+  // rate once work fills the chip, this one wastes neither border rows nor, on fewer tiles, so
+  // many splits.  The work counts padded channels.  us, window kernels / this one: 128ch
+  // 40 x 36 x 36 (15 GFLOP) 36.4 / 29.9, 26 x 66 x 66 (33) 60.4 / 55.6, 64 -> 256 on 40 x 72 x 72
+  // (61) 85.1 / 96.1, 16 -> 512 on 64 x 64 x 64 (155) 155 / 210; up to 64 output channels
+  // 160 x 64 x 64 (48) 88.7 / 75.1, 64 x 128 x 128 (77) 138 / 144; 512ch 128 x 8 x 8 (39, 1.4 rows
+  // per pixel) 72.6 / 58.7, 1024 x 8 x 8 380 / 431; half border, 4096 x 4 x 4 (309) 536 / 438.
+  const PxWgradPlan p = conv_px_wgrad_plan(kPxStride1, B, cin, cout, H, W, 0);
+  const double gflop = 2.0 * 9.0 * double(p.N) * p.ci_pad * p.co_pad * 1e-9;
+  const double border = double(conv_geom(B, H, W, layout).m_total) / p.N;
+  return border >= 1.8 || gflop <= (cout <= 64 ? 50.0 : 34.0) * border;
 }
 
 size_t xdna_conv3x3_px_wgrad_workspace_bytes(int form, int B, int Cin, int Cout, int H, int W) {
-  if (B < 1 || Cin < 1 || Cout < 1 || H < 1 || W < 1 || (form != kPxStride1 && form != kPxStride2)) return 0;
+  if (B < 1 || Cin < 1 || Cout < 1 || H < 1 || W < 1 || (form != kPxStride1 && form != kPxStride2) ||
+      !conv_px_wgrad_fits(form, B, Cin, Cout, H, W, kLayoutTight))
+    return 0;
   const PxWgradPlan p = conv_px_wgrad_plan(form, B, Cin, Cout, H, W, g_wgrad_splits.load());
   return align256(p.part_bytes) + align256(p.bpart_bytes);
 }
@@ -3556,7 +3562,7 @@ int xdna_conv3x3_px_wgrad_bf16(int form, const uint16_t* xp, const uint16_t* dp,
                                void* stream) {
   if (!shape_ok("xdna_conv3x3_px_wgrad_bf16", B, Cin, Cout, H, W)) return -1;
   if ((form != kPxStride1 && form != kPxStride2) || (layout != kLayoutRef && layout != kLayoutTight) ||
-      !conv_px_fits(form, B, Cin, Cout, H, W, layout) || !conv_px_fits(kPxStride1, B, Cout, Cin, H, W, layout)) {
+      !conv_px_wgrad_fits(form, B, Cin, Cout, H, W, layout)) {
     set_error("xdna_conv3x3_px_wgrad_bf16: unknown form or layout, or operands too large");
     return -1;
   }

@@ -31,6 +31,8 @@ struct PxWgradPlan {
   int N = 0, MC = 1, ci_pad = 0, co_pad = 0, kt_per = 0, splits = 0;
   size_t part_bytes = 0, bpart_bytes = 0;
 };
+// Whether the operands fit the offsets and the pixels a plan (2.6 million).
+bool conv_px_wgrad_fits(int form, int B, int Cin, int Cout, int H, int W, int layout);
 PxWgradPlan conv_px_wgrad_plan(int form, int B, int Cin, int Cout, int H, int W, int forced_splits);
 int conv_px_wgrad(const PxWgradPlan& p, int form, const uint16_t* xp, const uint16_t* dp, float* part, float* bpart, int B,
                   int Cin, int Cout, int H, int W, int layout, hipStream_t st);

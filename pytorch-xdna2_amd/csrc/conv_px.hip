@@ -326,6 +326,7 @@ constexpr int kPwK = 32;                   // pixels per k-tile
 constexpr int kPwTile = kPwK * 64;         // elements of a [32][64] tile
 constexpr int kPwStages = 3;
 constexpr int kPwMaxKt = 80;               // k-tiles per split: the table beside the ring leaves two workgroups per CU
+constexpr int kPwMaxSplits = 1024;
 constexpr int kPwOob = 0x7FFFFE00;         // a row past both operands: the DMA writes zeros
 
 // 16-byte piece q of pixel row r sits at q ^ 4 ((r >> 1) & 1): the four rows x 64 bytes of a
@@ -580,6 +581,14 @@ int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bi
   return rc;
 }
 
+bool conv_px_wgrad_fits(int form, int B, int Cin, int Cout, int H, int W, int layout) {
+  const int Ho = form == kPxStride2 ? (H + 1) / 2 : H, Wo = form == kPxStride2 ? (W + 1) / 2 : W;
+  // (dY's packed rows are the operand of a stride-1 conv of it; a split's table holds kPwMaxKt
+  // k-tiles, so more pixels than kPwMaxSplits of them have no plan)
+  return conv_px_fits(form, B, Cin, Cout, H, W, layout) && conv_px_fits(kPxStride1, B, Cout, Cin, H, W, layout) &&
+         ceil_div(int64_t(B) * Ho * Wo, kPwK) <= int64_t(kPwMaxSplits) * kPwMaxKt;
+}
+
 PxWgradPlan conv_px_wgrad_plan(int form, int B, int Cin, int Cout, int H, int W, int forced_splits) {
   PxWgradPlan p;
   const int Ho = form == kPxStride2 ? (H + 1) / 2 : H, Wo = form == kPxStride2 ? (W + 1) / 2 : W;
@@ -596,7 +605,7 @@ PxWgradPlan conv_px_wgrad_plan(int form, int B, int Cin, int Cout, int H, int W,
   // workgroup 2 us of prologue and epilogue, and the partials are written and read once.
   int64_t best = 1;
   double best_t = 1e30;
-  for (int64_t s = 1; s <= std::min<int64_t>(ktiles, 1024); s += s < 32 ? 1 : 8) {
+  for (int64_t s = 1; s <= std::min<int64_t>(ktiles, kPwMaxSplits); s += s < 32 ? 1 : 8) {
     const int64_t kt = ceil_div(ktiles, s);
     if (kt > kPwMaxKt) continue;
     const double per_cu = double(s % 8 ? ceil_div(tiles * s, 256) : ceil_div(s / 8 * tiles, 32));

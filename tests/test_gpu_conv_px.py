@@ -110,6 +110,13 @@ def test_pick(hip):
     assert pick(3, 40, 128, 128, 9, 9, 1) == 1
     assert pick(1, 4096, 512, 64, 64, 64, 1) == 0  # more than 2 GiB of packed rows
     assert hip.xdna_conv3x3_px_bf16(1, 1, 1, None, 1, 4096, 512, 64, 64, 64, 1, 0, 0, stream()) == -1
+    assert pick(3, 160, 64, 64, 64, 64, 1) == 1 and pick(3, 64, 64, 512, 64, 64, 1) == 0
+    assert pick(3, 128, 512, 512, 8, 8, 1) == 1 and pick(3, 1024, 512, 512, 8, 8, 1) == 0
+    # the weight gradient: more pixels than its splits hold
+    assert pick(4, 40, 16, 16, 512, 512, 1) == 1 and pick(4, 41, 16, 16, 512, 512, 1) == 0
+    ws = hip.xdna_conv3x3_px_wgrad_workspace_bytes
+    assert ws(0, 40, 64, 64, 256, 256) > 0 and ws(0, 64, 64, 64, 256, 256) == 0
+    assert hip.xdna_conv3x3_px_wgrad_bf16(0, 1, 1, 1, None, 64, 64, 64, 256, 256, 1, 1, 1 << 40, stream()) == -1
     assert hip.xdna_conv3x3_set_rows_variant(9) == 0
     assert pick(1, 128, 64, 128, 64, 64, 1) == 0
     assert hip.xdna_conv3x3_set_rows_variant(0) == 0
