@@ -3537,16 +3537,17 @@ int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int lay
     return cin > 3 * kKStep && ceil_div(g.m_total, 256) * ceil_div(cout, kSCo) < 150;
   }
   // the weight gradient, on `border` packed rows per pixel: the window kernels have the higher
-  // rate once work fills the chip, this one wastes neither border rows nor, on fewer tiles, so
-  // many splits.  The work counts padded channels.  us, window kernels / this one: 128ch
-  // 40 x 36 x 36 (15 GFLOP) 36.4 / 29.9, 26 x 66 x 66 (33) 60.4 / 55.6, 64 -> 256 on 40 x 72 x 72
-  // (61) 85.1 / 96.1, 16 -> 512 on 64 x 64 x 64 (155) 155 / 210; up to 64 output channels
-  // 160 x 64 x 64 (48) 88.7 / 75.1, 64 x 128 x 128 (77) 138 / 144; 512ch 128 x 8 x 8 (39, 1.4 rows
-  // per pixel) 72.6 / 58.7, 1024 x 8 x 8 380 / 431; half border, 4096 x 4 x 4 (309) 536 / 438.
+  // rate once work fills the chip (1.2 against 0.87 PFLOP/s), this one wastes neither border
+  // rows nor, on fewer tiles, so many splits.  The work counts padded channels.  us, window
+  // kernels / this one: 128ch 40 x 36 x 36 (15 GFLOP) 36.4 / 29, 256ch 40 x 36 x 36 (61) 81.8 /
+  // 76.5, 128 -> 256 on 64 x 48 x 48 (87) 108 / 106, 256ch 64 x 36 x 36 (98) 116 / 119, 512ch
+  // 64 x 36 x 36 (391) 355 / 451, 16 -> 512 on 64 x 64 x 64 (155) 166 / 175; up to 64 output channels
+  // (half the work per load) 160 x 64 x 64 (48) 88.7 / 76.9, 64 x 128 x 128 (77) 138 / 144; 512ch
+  // 1024 x 8 x 8 (309, 1.57 rows per pixel) 400 / 349, 4096 x 4 x 4 566 / 351.
   const PxWgradPlan p = conv_px_wgrad_plan(kPxStride1, B, cin, cout, H, W, 0);
   const double gflop = 2.0 * 9.0 * double(p.N) * p.ci_pad * p.co_pad * 1e-9;
   const double border = double(conv_geom(B, H, W, layout).m_total) / p.N;
-  return border >= 1.8 || gflop <= (cout <= 64 ? 50.0 : 34.0) * border;
+  return border >= 1.55 || gflop <= (cout <= 64 ? 50.0 : 80.0) * border;
 }
 
 size_t xdna_conv3x3_px_wgrad_workspace_bytes(int form, int B, int Cin, int Cout, int H, int W) {

@@ -331,8 +331,12 @@ constexpr int kPwOob = 0x7FFFFE00;         // a row past both operands: the DMA 
 
 // 16-byte piece q of pixel row r sits at q ^ 4 ((r >> 1) & 1): the four rows x 64 bytes of a
 // half-wave's transposing read fall on 64 distinct banks.
+//
+// Two workgroups per CU (the second bound: 228 registers; left alone, MC 2 took 279 and one
+// workgroup, whose loads nothing covered): 64 -> 256 on 40 x 72 x 72 96 -> 82 us, 512ch
+// 1024 x 8 x 8 431 -> 349, 512ch 16 x 18 x 18 43.4 -> 38.3.
 template <int MC>
-__global__ __launch_bounds__(256) void px_wgrad_kernel(PxWgArgs a) {
+__global__ __launch_bounds__(256, 2) void px_wgrad_kernel(PxWgArgs a) {
   constexpr int kTiles = MC + 3;           // [32][64] tiles per k-tile: dY's, one per tap
   constexpr int kStage = kTiles * kPwTile;
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];

@@ -111,7 +111,7 @@ def test_pick(hip):
     assert pick(1, 4096, 512, 64, 64, 64, 1) == 0  # more than 2 GiB of packed rows
     assert hip.xdna_conv3x3_px_bf16(1, 1, 1, None, 1, 4096, 512, 64, 64, 64, 1, 0, 0, stream()) == -1
     assert pick(3, 160, 64, 64, 64, 64, 1) == 1 and pick(3, 64, 64, 512, 64, 64, 1) == 0
-    assert pick(3, 128, 512, 512, 8, 8, 1) == 1 and pick(3, 1024, 512, 512, 8, 8, 1) == 0
+    assert pick(3, 1024, 512, 512, 8, 8, 1) == 1 and pick(3, 64, 512, 512, 36, 36, 1) == 0
     # the weight gradient: more pixels than its splits hold
     assert pick(4, 40, 16, 16, 512, 512, 1) == 1 and pick(4, 41, 16, 16, 512, 512, 1) == 0
     ws = hip.xdna_conv3x3_px_wgrad_workspace_bytes
