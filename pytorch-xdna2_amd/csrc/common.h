@@ -136,6 +136,10 @@ struct __attribute__((packed, aligned(2))) Pix4 {
   uint32_t lo, hi;
 };
 
+struct __attribute__((packed, aligned(2))) Pix2 {
+  uint32_t v;
+};
+
 struct __attribute__((packed, aligned(2))) Pix8 {
   uint32_t v[4];
 };

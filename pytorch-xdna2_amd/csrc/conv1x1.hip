@@ -29,10 +29,6 @@
 namespace xdna {
 namespace {
 
-struct __attribute__((packed, aligned(2))) Pix2 {
-  uint32_t v;
-};
-
 struct C1Args {
   const uint16_t* x;     // the input of this direction
   const uint16_t* w;     // [Cout][Cin] of the conv

@@ -21,7 +21,8 @@ bool conv_px_fits(int form, int B, int cin, int cout, int H, int W, int layout);
 
 // y (or, kPxS2Dgrad, dx) = act(conv + bias).  xp: packed rows of `layout`; wt: the prepared
 // weights [co_pad][chunks * 9 * 64].  tile: 0 automatic; 1 64 x 64 (channels x pixels),
-// K split over the waves; 2 64 x 64; 3 64 x 128; 4 128 x 128 (measurements).  0 when launched, -1 with the error set.
+// K split over the waves; 2 64 x 64; 3 64 x 128; 4 128 x 128; kPxS2Dgrad in column pairs
+// 5 64 x 64, 6 64 x 128 (measurements).  0 when launched, -1 with the error set.
 int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bias, uint16_t* out, int B, int cin,
             int cout, int H, int W, int layout, int act, int tile, hipStream_t st);
 

@@ -75,7 +75,11 @@ __device__ inline void px_pixel(const PxArgs& a, int phase, int n, int& b, int& 
 // whole tile over a quarter of every k-tile (k-step = wave) and the four partial tiles are
 // added in wave order through LDS: every fragment is read once per workgroup instead of
 // twice, and consecutive MFMAs are independent, for one exchange per tile.
-template <int MI, int NJ, int NS, int KW>
+//
+// kPair (the stride-2 input gradient, KW 1): a workgroup multiplies both column parities of its
+// lattice pixels, one after the other on one ring, and stores them as pairs.  One parity alone
+// stores every other pixel, 2 bytes each: half lines, written twice.
+template <int MI, int NJ, int NS, int KW, bool kPair>
 __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
   constexpr int TM = 64 * MI, TN = 64 * NJ;
   constexpr int kStage = (TM + TN) * 64;          // elements of one k-tile
@@ -84,7 +88,7 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
   const int lr = lane & 31, half = lane >> 5;
-  const int phase = blockIdx.y, split = blockIdx.z;
+  const int phase = kPair ? 2 * blockIdx.y : blockIdx.y, split = blockIdx.z;
   // XCD x (workgroup L on XCD L % 8) takes every channel tile of its pixel tiles
   const int L = blockIdx.x, k8 = L >> 3;
   const int pt = (k8 / a.nct) * 8 + (L & 7), ct = k8 % a.nct;
@@ -92,9 +96,9 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
   const int n0 = pt * TN, co0 = ct * TM;
   if (n0 >= N) return;
 
-  const PxTaps& taps = a.taps[phase];
   const int c_beg = split * a.ch_per, c_end = min(a.chunks, c_beg + a.ch_per);
-  const int nkt = (c_end - c_beg) * taps.n;
+  const int nkt = (c_end - c_beg) * a.taps[phase].n;
+  const int nkt1 = kPair ? (c_end - c_beg) * a.taps[phase + 1].n : 0;  // the odd columns'
   const i32x4_t rsw = uniform_rsrc(lds_dma_rsrc(a.wt, a.w_bytes)), rsx = uniform_rsrc(lds_dma_rsrc(a.xp, a.x_bytes));
   // this wave's DMA blocks of 8 rows: lane L at row 8 blk + L / 8, position L % 8
   int va[2 * MI], vb[2 * NJ];
@@ -117,8 +121,8 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
   }
   const uint32_t lds0 = lds_addr(smem);
   // the k-tile to issue next; past the last one it stays there (its loads are never read)
-  int ic = c_beg, it = 0, in = 0;
-  int soa = (ic * 9 + taps.w[0]) * 128, sob = (ic * kGroupRows + taps.off[0]) * 128;
+  int ic = c_beg, it = 0, in = 0, iph = phase;
+  int soa = (ic * 9 + a.taps[iph].w[0]) * 128, sob = (ic * kGroupRows + a.taps[iph].off[0]) * 128;
   auto issue = [&](int slot, int q) {
     const uint32_t m0 = lds0 + uint32_t(slot * kStage * 2);
     if (q < 2 * MI)
@@ -127,13 +131,17 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
       lds_dma16_soff(rsx, m0 + uint32_t(TM * 128 + (wave * 2 * NJ + q - 2 * MI) * 1024), vb[q < 2 * MI ? 0 : q - 2 * MI], sob);
   };
   auto issued = [&] {
-    if (++in < nkt) {
-      if (++it == taps.n) {
+    if (++in < nkt + nkt1) {
+      if (++it == a.taps[iph].n) {
         it = 0;
         ++ic;
+        if (kPair && ic == c_end) {
+          ic = c_beg;
+          iph = phase + 1;
+        }
       }
-      soa = (ic * 9 + taps.w[it]) * 128;
-      sob = (ic * kGroupRows + taps.off[it]) * 128;
+      soa = (ic * 9 + a.taps[iph].w[it]) * 128;
+      sob = (ic * kGroupRows + a.taps[iph].off[it]) * 128;
     }
   };
 #pragma unroll
@@ -145,11 +153,14 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
 
   constexpr int BI = KW == 4 ? 2 * MI : MI, BJ = KW == 4 ? 2 * NJ : NJ;  // blocks a wave multiplies
   constexpr int KS = KW == 4 ? 1 : 4;                                    // k-steps of a k-tile it takes
-  f32x16_t acc[BI][BJ];
+  f32x16_t acc[BI][BJ], acc1[kPair ? BI : 1][kPair ? BJ : 1];
 #pragma unroll
   for (int i = 0; i < BI; ++i)
 #pragma unroll
-    for (int j = 0; j < BJ; ++j) acc[i][j] = zero_acc();
+    for (int j = 0; j < BJ; ++j) {
+      acc[i][j] = zero_acc();
+      if (kPair) acc1[kPair ? i : 0][kPair ? j : 0] = zero_acc();
+    }
   float bias[MI][16];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
@@ -176,7 +187,7 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
   // k-tile t from `cur`, read before; k-tile t + 1's fragments into `nxt` and the loads of
   // k-tile t + NS into this one's slot between the MFMAs
   int slot = 0;
-  auto ktile = [&](const Frags& cur, Frags& nxt) {
+  auto ktile = [&](const Frags& cur, Frags& nxt, auto& sum) {
     lds_reads_wait();                     // this wave's reads of k-tile t are done: its slot is free
     lds_dma_wait<(NS - 2) * kLoads>();    // this wave's loads of k-tile t + 1 have landed
     __builtin_amdgcn_s_barrier();
@@ -189,7 +200,7 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
       for (int i = 0; i < BI; ++i)
 #pragma unroll
         for (int j = 0; j < BJ; ++j) {
-          acc[i][j] = mfma_32x32x16(as_bf16x8(cur.a[ks][i]), as_bf16x8(cur.b[ks][j]), acc[i][j]);
+          sum[i][j] = mfma_32x32x16(as_bf16x8(cur.a[ks][i]), as_bf16x8(cur.b[ks][j]), sum[i][j]);
           if (i == 0 && j == 0) read(nxt, next, ks);
           constexpr int kPer = (kLoads + KS * BI * BJ - 1) / (KS * BI * BJ);
 #pragma unroll
@@ -210,8 +221,15 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) read(f0, 0, ks);
   for (int t = 0; t < nkt; t += 2) {
-    ktile(f0, f1);
-    if (t + 1 < nkt) ktile(f1, f0);
+    ktile(f0, f1, acc);
+    if (t + 1 < nkt) ktile(f1, f0, acc);
+  }
+  if constexpr (kPair) {
+    if (nkt & 1) f0 = f1;
+    for (int t = 0; t < nkt1; t += 2) {
+      ktile(f0, f1, acc1);
+      if (t + 1 < nkt1) ktile(f1, f0, acc1);
+    }
   }
   lds_dma_wait<0>();
   if constexpr (KW == 4) {
@@ -255,6 +273,23 @@ __global__ __launch_bounds__(256) void conv_px_kernel(PxArgs a) {
     int b, y, x;
     px_pixel(a, phase, min(n, N - 1), b, y, x);
     const int plane = a.oH * a.oW;
+    if constexpr (kPair) {
+      uint16_t* o = a.out + int64_t(b) * a.cout * plane + (2 * y + (phase >> 1)) * a.oW + 2 * x;
+      const bool both = 2 * x + 1 < a.oW;  // (an odd width's last column has no odd neighbour)
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int co = co0 + (wm * MI + i) * 32 + mfma_row(r, lane);
+          if (n >= N || co >= a.cout) continue;
+          const uint32_t lo = f32_to_bf16(act_forward(a.act, 0.0f, acc[i][j][r] + bias[i][r]));
+          const uint32_t hi = f32_to_bf16(act_forward(a.act, 0.0f, acc1[i][j][r] + bias[i][r]));
+          uint16_t* p = o + int64_t(co) * plane;
+          if (both) *reinterpret_cast<Pix2*>(p) = Pix2{lo | (hi << 16)};
+          else *p = uint16_t(lo);
+        }
+      continue;
+    }
     const int po =
         n < N ? (b * a.cout * plane + (y * a.os + (phase >> 1)) * a.oW + x * a.os + (phase & 1)) * 2 : kPxSkip;
 #pragma unroll
@@ -281,11 +316,11 @@ __global__ __launch_bounds__(256) void px_reduce_kernel(PxArgs a) {
   a.out[(int64_t(b) * a.cout + co) * plane + pix] = f32_to_bf16(act_forward(a.act, 0.0f, v));
 }
 
-template <int MI, int NJ, int NS, int KW>
+template <int MI, int NJ, int NS, int KW, bool kPair = false>
 int launch_px(PxArgs a, int phases, hipStream_t st) {
   constexpr int kRing = NS * (64 * MI + 64 * NJ) * 64 * 2, kRed = KW == 4 ? 4 * 64 * MI * 64 * NJ * 4 : 0;
   constexpr int kLds = kRing > kRed ? kRing : kRed;
-  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_px_kernel<MI, NJ, NS, KW>),
+  static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_px_kernel<MI, NJ, NS, KW, kPair>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, kLds) == hipSuccess;
   if (!ok) {
     set_error("conv3x3 pixels: cannot enable the kernel's LDS size");
@@ -294,7 +329,7 @@ int launch_px(PxArgs a, int phases, hipStream_t st) {
   a.npt = int(ceil_div(*std::max_element(a.N, a.N + 4), 64 * NJ));
   a.nct = int(ceil_div(a.cout, 64 * MI));
   const dim3 grid(unsigned(ceil_div(a.npt, 8) * 8 * a.nct), unsigned(phases), unsigned(a.nsplit));
-  conv_px_kernel<MI, NJ, NS, KW><<<grid, 256, kLds, st>>>(a);
+  conv_px_kernel<MI, NJ, NS, KW, kPair><<<grid, 256, kLds, st>>>(a);
   if (a.part) px_reduce_kernel<<<dim3(unsigned(ceil_div(a.N[0], 256)), unsigned(a.cout)), 256, 0, st>>>(a);
   return check_launch("conv3x3 pixels");
 }
@@ -552,15 +587,26 @@ int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bi
   a.ch_per = a.chunks;
   const int64_t wgs = ceil_div(a.N[0], 64) * ceil_div(cout, 64);
   if (tile == 0) {
-    // 128 x 128 tiles, then 64 x 128, where they give two workgroups per CU (the input
-    // gradient of 128 -> 64 channels at 128 x 64 x 64: 64 x 128 67 us, 128 x 128 96, 64 x 64
-    // 76); below, 64 x 64, the waves splitting K from 36 k-tiles on (326 channels, 11 x 13 x 13:
-    // 15.2 against 17.2 us)
-    const int64_t wide = ceil_div(a.N[0], 128) * phases;
+    // 128 x 128 tiles, then 64 x 128, where they give two workgroups per CU; below, 64 x 64, the
+    // waves splitting K from 36 k-tiles on (326 channels, 11 x 13 x 13: 15.2 against 17.2 us).
+    // The input gradient in column pairs where half as many, longer workgroups still cover
+    // the chip: 64 x 128 from 320 of them on (us, without / with pairs: 128 -> 64 channels on
+    // 128 x 64 x 64 72 / 57, on 24 x 61 x 67 22 / 17, 32 -> 16 on 16 x 72 x 72 13.1 / 9.7), 64 x 64 from
+    // 400 (64 -> 32 on 40 x 36 x 36 10.1 / 8.4; 128 -> 64 on 40 x 18 x 18, 102 of them, 6.9 / 9.0).
+    // 128 x 128 leaves no registers for a pair's sums and wins on weights read once (512 -> 512
+    // on 64 x 24 x 24 73 / 80).
+    const int64_t wide = ceil_div(a.N[0], 128) * phases, ct = ceil_div(cout, 64);
+    const bool dx = form == kPxS2Dgrad;
     tile = cout > 64 && wide * ceil_div(cout, 128) >= 512 ? 4
-           : wide * ceil_div(cout, 64) >= 512             ? 3
+           : dx && ceil_div(a.N[0], 128) * 2 * ct >= 320  ? 6
+           : dx && ceil_div(a.N[0], 64) * 2 * ct >= 400   ? 5
+           : wide * ct >= 512                             ? 3
            : a.chunks * a.taps[phases - 1].n >= 36        ? 1
                                                           : 2;
+  }
+  if (tile > 4 && form != kPxS2Dgrad) {
+    set_error("conv3x3 pixels: tiles 5 and 6 are the stride-2 input gradient's");
+    return -1;
   }
   // one lattice of few 64 x 64 tiles: K split over workgroups, at least 18 k-tiles each (the
   // reduce costs what 10 take)
@@ -578,7 +624,9 @@ int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bi
     case 1: rc = launch_px<1, 1, 4, 4>(a, phases, st); break;
     case 2: rc = launch_px<1, 1, 4, 1>(a, phases, st); break;
     case 3: rc = launch_px<1, 2, 3, 1>(a, phases, st); break;
-    default: rc = launch_px<2, 2, 2, 1>(a, phases, st); break;
+    case 4: rc = launch_px<2, 2, 2, 1>(a, phases, st); break;
+    case 5: rc = launch_px<1, 1, 4, 1, true>(a, 2, st); break;
+    default: rc = launch_px<1, 2, 3, 1, true>(a, 2, st); break;
   }
   // stream-ordered reuse: the next user of the block runs after the reduce
   if (a.part) xdna_hip_cache_free(a.part);
