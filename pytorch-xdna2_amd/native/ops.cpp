@@ -64,12 +64,11 @@ bool conv_eligible(const at::Tensor& x, const at::Tensor& w, c10::SymIntArrayRef
   return true;
 }
 
-// 3x3 / stride-2 / pad-1 convs (the style encoder, ResNet's downsampling blocks) run
-// through the stride-1 kernels: the forward is the stride-1 conv at every other row and
-// column, and both gradients are the stride-1 ones of the gradient spread onto the
-// stride-1 grid with zeros (which add nothing to any sum), so the numerics are those of
-// the hot path.  4x the MACs of the strided conv, on kernels several times faster than
-// MIOpen's on these shapes, and within the conv bar where MIOpen is not.  The reference
+// 3x3 / stride-2 / pad-1 convs (the style encoder, ResNet's downsampling blocks) run on the
+// real-pixel kernels (xdna_conv3x3_px_*) on the stride-1 path's packed rows and prepared
+// weights.  Operands past those kernels' 32-bit offsets, and runs that force a stride-1
+// kernel, take the stride-1 form: the conv at every other row and column, and the gradients
+// of the output gradient spread onto the stride-1 grid with zeros (4x the MACs).  The reference
 // runs them on its CPU through the fallback (torch_xdna_device.cpp:4524-4606, 4608-4885).
 // XDNA_CONV_S2=0 sends 3x3 / stride-2 convs to the general kernels instead (their real
 // MACs on the gather GEMM), for measurements.
@@ -1256,8 +1255,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
                      grad_output.size(1) == weight.size(0) && grad_output.size(0) == input.size(0);
   bool hip = conv_eligible(input, weight, stride, padding, dilation, transposed, output_padding, groups) &&
              go_ok && grad_output.size(2) == input.size(2) && grad_output.size(3) == input.size(3);
-  // stride 2: the stride-1 gradients of the gradient spread onto the stride-1 grid
-  // stride 2: the stride-1 gradients of the gradient spread onto the stride-1 grid (its
+  // stride 2 beside the real-pixel kernels: the stride-1 gradients of the gradient spread onto the stride-1 grid (its
   // packed rows made in one pass; the spread tensor itself only for the channel-major
   // weight gradient)
   at::Tensor go = grad_output;
