@@ -366,8 +366,8 @@ int xdna_conv3x3_layout_rows_bf16(const uint16_t* xp, const uint16_t* wt, const 
  * forward of 3x3 / stride 2 / pad 1 (y ceil(H/2) x ceil(W/2)) from the packed rows of x; 2: that
  * conv's input gradient (y H x W) from the packed rows of the ceil(H/2) x ceil(W/2) gradient and
  * the input gradient's prepared weights, cin and cout being the gradient's and x's channels.
- * act as above; tile 0 automatic (others for measurements).  Returns -1 for operands past
- * 32-bit offsets. */
+ * act as above; tile 0 automatic, 1-4 (form 2: 1-6) for measurements.  xp and wt 16-byte aligned.
+ * Returns -1 for operands past 32-bit offsets and for any other tile. */
 int xdna_conv3x3_px_bf16(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bias, uint16_t* y, int B,
                          int cin, int cout, int H, int W, int layout, int act, int tile, void* stream);
 

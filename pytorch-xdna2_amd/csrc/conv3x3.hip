@@ -2070,6 +2070,13 @@ bool shape_ok(const char* what, int B, int Cin, int Cout, int H, int W) {
   return true;
 }
 
+// The packed rows and prepared weights reach LDS by 16-byte DMA.
+bool px_operands_ok(const char* what, const void* a, const void* b, const void* out) {
+  if (a && b && out && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0) return true;
+  set_error(std::string(what) + ": null operand, or packed rows or prepared weights not 16-byte aligned");
+  return false;
+}
+
 // The forward form (wt) and / or the input-gradient form (wtd) of an OIHW weight in one
 // launch of prep_tiled_kernel.
 // output-channel tile of the weight preparation: 0 by size, else 8 or 32
@@ -3516,6 +3523,12 @@ int xdna_conv3x3_px_bf16(int form, const uint16_t* xp, const uint16_t* wt, const
     set_error("xdna_conv3x3_px_bf16: unknown form, layout or activation, or operands too large");
     return -1;
   }
+  // (tiles 5 and 6 store column pairs of the stride-2 input gradient, past any other form's output)
+  if (tile < 0 || tile > (form == kPxS2Dgrad ? 6 : 4)) {
+    set_error("xdna_conv3x3_px_bf16: unknown tile for this form");
+    return -1;
+  }
+  if (!px_operands_ok("xdna_conv3x3_px_bf16", xp, wt, y)) return -1;
   if (!admit_launch("xdna_conv3x3_px_bf16")) return -1;
   return conv_px(form, xp, wt, bias, y, B, cin, cout, H, W, layout, act, tile, as_stream(stream));
 }
@@ -3567,9 +3580,11 @@ int xdna_conv3x3_px_wgrad_bf16(int form, const uint16_t* xp, const uint16_t* dp,
     set_error("xdna_conv3x3_px_wgrad_bf16: unknown form or layout, or operands too large");
     return -1;
   }
+  if (!px_operands_ok("xdna_conv3x3_px_wgrad_bf16", xp, dp, gw)) return -1;
   const PxWgradPlan p = conv_px_wgrad_plan(form, B, Cin, Cout, H, W, g_wgrad_splits.load());
-  if (!workspace || workspace_bytes < align256(p.part_bytes) + align256(p.bpart_bytes)) {
-    set_error("xdna_conv3x3_px_wgrad_bf16: workspace too small");
+  if (!workspace || workspace_bytes < align256(p.part_bytes) + align256(p.bpart_bytes) ||
+      (reinterpret_cast<uintptr_t>(workspace) & 3)) {
+    set_error("xdna_conv3x3_px_wgrad_bf16: workspace too small or not 4-byte aligned");
     return -1;
   }
   if (!admit_launch("xdna_conv3x3_px_wgrad_bf16")) return -1;

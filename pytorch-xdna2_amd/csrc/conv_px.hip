@@ -604,10 +604,6 @@ int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bi
            : a.chunks * a.taps[phases - 1].n >= 36        ? 1
                                                           : 2;
   }
-  if (tile > 4 && form != kPxS2Dgrad) {
-    set_error("conv3x3 pixels: tiles 5 and 6 are the stride-2 input gradient's");
-    return -1;
-  }
   // one lattice of few 64 x 64 tiles: K split over workgroups, at least 18 k-tiles each (the
   // reduce costs what 10 take)
   const int ns = int(std::min<int64_t>(256 / std::max<int64_t>(wgs, 1), a.chunks / 2));
@@ -626,7 +622,8 @@ int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bi
     case 3: rc = launch_px<1, 2, 3, 1>(a, phases, st); break;
     case 4: rc = launch_px<2, 2, 2, 1>(a, phases, st); break;
     case 5: rc = launch_px<1, 1, 4, 1, true>(a, 2, st); break;
-    default: rc = launch_px<1, 2, 3, 1, true>(a, 2, st); break;
+    case 6: rc = launch_px<1, 2, 3, 1, true>(a, 2, st); break;
+    default: set_error("conv3x3 pixels: unknown tile"); rc = -1;
   }
   // stream-ordered reuse: the next user of the block runs after the reduce
   if (a.part) xdna_hip_cache_free(a.part);

@@ -43,6 +43,30 @@ def test_invalid_arguments_report_errors():
     assert lib.xdna_conv3x3w_pack_input_bf16(None, None, 0, 3, 4, 4, 1, None) == 0
 
 
+def test_px_conv_refuses_bad_arguments():
+    """A tile outside a form's range (the pair tiles' stores fit the stride-2 input gradient only),
+    a null or misaligned operand: refused on the host, with its reason, before any launch."""
+    lib = hip_abi.load()
+    good = [0x1000, 0x1000, None, 0x1000]  # never dereferenced
+
+    def refused(form, operands, tile, why):
+        rc = lib.xdna_conv3x3_px_bf16(form, *operands, 2, 64, 64, 8, 8, 1, 0, tile, None)
+        return rc == -1 and why in hip_abi.last_error()
+
+    for form, tiles in ((0, (-1, 5, 6, 7)), (1, (-1, 5, 6, 7)), (2, (-1, 7, 100))):
+        for t in tiles:
+            assert refused(form, good, t, "unknown tile"), (form, t, hip_abi.last_error())
+        for i in (0, 1, 3):
+            assert refused(form, good[:i] + [None] + good[i + 1:], 0, "null operand"), (form, i)
+        for i in (0, 1):
+            assert refused(form, good[:i] + [0x1008] + good[i + 1:], 0, "aligned"), (form, i)
+    need = lib.xdna_conv3x3_px_wgrad_workspace_bytes(0, 2, 64, 64, 8, 8)
+    for ops, ws, why in ([(None, 0x1000, 0x1000), 0x1000, "null"], [(0x1000, 0x1004, 0x1000), 0x1000, "aligned"],
+                         [(0x1000, 0x1000, None), 0x1000, "null"], [(0x1000, 0x1000, 0x1000), 0x1002, "workspace"]):
+        rc = lib.xdna_conv3x3_px_wgrad_bf16(0, *ops, None, 2, 64, 64, 8, 8, 1, ws, need, None)
+        assert rc == -1 and why in hip_abi.last_error(), (ops, ws, hip_abi.last_error())
+
+
 def test_geometry_matches_reference_plan():
     lib = hip_abi.load()
     out = (hip_abi.L * 7)()
