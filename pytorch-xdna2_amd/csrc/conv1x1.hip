@@ -26,6 +26,8 @@
 #include "mfma.h"
 #include "../../include/xdna_hip.h"
 
+#include <algorithm>
+
 namespace xdna {
 namespace {
 
@@ -344,6 +346,8 @@ __global__ __launch_bounds__(256) void conv1x1_wgrad_reduce_kernel(const float* 
   gw[e] = f32_to_bf16(s);
 }
 
+constexpr int64_t kMaxGridX = (int64_t(1) << 24) - 1;  // workgroups of 256 threads: a grid side under 2^32 threads
+
 struct C1Geom {
   int Ho, Wo, P;
 };
@@ -383,7 +387,7 @@ int c1_launch(const char* who, bool dx, const uint16_t* x, const uint16_t* w, co
   const bool narrow = c1_narrow(g.M);
   g.tpi = int(ceil_div(q.P, narrow ? 128 : 64));
   const int64_t gx = int64_t(B) * g.tpi, gy = ceil_div(g.M, narrow ? 64 : 128);
-  if (gx > 0x7FFFFFFF || gy > 65535) {
+  if (gx > kMaxGridX || gy > 65535) {
     set_error(std::string(who) + ": grid too large");
     return -1;
   }
@@ -428,6 +432,64 @@ C1WgPlan c1_wgrad_plan(int B, int Cin, int Cout, int P) {
   return p;
 }
 
+// Modelled times, us, of these kernels and of the products they stand beside, fitted to 2500
+// random shapes (1 - 256 images, 4 - 2048 channels, planes from 1 x 1 to 100 x 100, both strides;
+// 20 - 30 % off at one standard deviation).  A workgroup is a chain of ceil(K / 64) rounds of about
+// one load latency each, so a long k on few workgroups belongs to the GEMM, whose k groups and
+// splits cut the chain (512 -> 64 stride 2 on 39 x 7 x 10: 53 in place, 12 as a product; input
+// gradient of 85 -> 2048 on 12 x 2 x 2: 101 / 13.5), and many workgroups, or planes whose
+// pixels fill no GEMM tile, belong here (64 -> 128 stride 2 on 128 x 64 x 64 19 / 37; input gradient
+// of 1024 -> 1483 on 190 x 4 x 2 81 / 275).  For less than two workgroups per CU; the choice asks for 12 % in favour of these kernels.
+double c1_mb(int64_t elements) { return 2e-6 * double(elements); }
+
+// rows beyond the first that 8 consecutive pixels of the strided plane touch
+int c1_row_breaks(const C1Geom& q) { return std::min(int(ceil_div(8, std::min(q.Wo, 8))), q.Ho) - 1; }
+
+// forward / input gradient, `wgs` workgroups of M outputs over K
+double c1_us(bool dx, int64_t wgs, int B, int M, int K, int Cin, int H, int W, const C1Geom& q, int stride) {
+  const double rounds = double(ceil_div(K, 64)), waves = std::max(1.0, double(wgs) / 256);
+  const bool narrow = c1_narrow(M), odd_px = q.P % 8 != 0, s2 = stride == 2;
+  const double mb = c1_mb(int64_t(B) * q.P * (M + K) + int64_t(M) * K);
+  if (!dx) {
+    const double round = 0.92 + 0.52 * narrow + 0.40 * odd_px + 0.28 * (K % 8 != 0) + s2 * (0.28 + 0.49 * c1_row_breaks(q));
+    return 3.8 + rounds * round * (1 + 0.54 * (waves - 1)) + 0.22 * mb;
+  }
+  const double round = 1.1 + 0.29 * narrow + 0.45 * odd_px + 1.0 * (M % 8 != 0);
+  // a spread piece that crosses a row's end is stored pixel by pixel
+  const double crossing = q.Wo % 8 == 0 ? 0.0 : std::min(1.5, 8.0 / q.Wo);
+  return 3.8 + rounds * round * (1 + 0.34 * (waves - 1)) + 0.19 * mb +
+         s2 * (1.1 * waves + (0.22 + 0.8 * crossing) * c1_mb(int64_t(B) * Cin * H * W));
+}
+
+// the batched product (and, stride 2, the sampling or spreading pass)
+double c1_gemm_us(bool dx, int B, int M, int K, int Cin, int H, int W, const C1Geom& q, int stride) {
+  const double rounds = double(ceil_div(K, 64)), tiles = double(B) * double(ceil_div(q.P, 64)) * double(ceil_div(M, 64));
+  const double gf = 2e-9 * B * double(q.P) * M * K, full = stride == 2 ? c1_mb(int64_t(B) * Cin * H * W) : 0.0;
+  const bool odd_px = q.P % 8 != 0, odd_w = Cin % 8 != 0, s2 = stride == 2;  // operands staged by elements
+  if (!dx)
+    return 4.9 + s2 * 2.1 + 0.42 * full + 2.0 * odd_px + 4.5 * odd_w + 2.2 * gf * (odd_px + odd_w) + 0.39 * std::min(rounds, 4.0) +
+           1.7 * tiles * rounds / 512;
+  return 3.8 + s2 * 1.7 + 1.1 * full + 2.0 * odd_px + 3.5 * odd_w + gf * (0.66 + 0.98 * (odd_px + odd_w)) +
+         0.81 * std::min(rounds, 4.0) + 2.0 * tiles * rounds / 512;
+}
+
+// weight gradient: a chain of 64-pixel steps, then the partials' sum (505 -> 1024 on 200 x 3 x 3, steps
+// of 9 pixels, loses: the product's copies are contiguous over images)
+double c1_wgrad_us(const C1WgPlan& p, int B, int Cin, int Cout, int H, int W, const C1Geom& q, int stride) {
+  const double step = 1.3 + 0.93 * (q.P % 8 != 0) + (stride == 2) * (0.72 + 0.86 * c1_row_breaks(q));
+  const double n = 1e-6 * Cin * double(Cout);
+  return 7.4 + p.per * step + 2.7 * p.nsplit * n + 3.1 * n + 0.09 * c1_mb(int64_t(B) * q.P * (Cin + Cout));
+}
+
+// channel-major copies (none of a single image) and one product over the pixels
+double c1_wgrad_gemm_us(int B, int Cin, int Cout, int H, int W, const C1Geom& q, int stride) {
+  const double k = double(B) * q.P, n = 1e-6 * Cin * double(Cout);
+  const double odd = int64_t(B) * q.P % 8 != 0, padded = 2e-9 * 128 * double(ceil_div(Cin, 128)) * 128 * double(ceil_div(Cout, 128)) * k;
+  return 7.2 + (stride == 2) * (2.0 + 0.38 * c1_mb(int64_t(B) * Cin * H * W)) +
+         (B > 1) * (7.8 + c1_mb(int64_t(B) * q.P * (Cin + Cout))) + 4.5e-3 * n * k * odd + 1.1 * n + 0.24 * std::min(k / 64, 16.0) +
+         5.9 * odd + 3.8 * padded;
+}
+
 }  // namespace
 }  // namespace xdna
 
@@ -444,27 +506,30 @@ int xdna_conv1x1_pick(int op, int B, int Cin, int Cout, int H, int W, int stride
   }
   if (!c1_geom("xdna_conv1x1_pick", &one, &one, &one, B, Cin, Cout, H, W, stride, q)) return -1;
   if (op == 2) {
-    // Many outputs from few pixels: 2 copies to channel-major rows and one product on 256 x 256
-    // tiles (us, this form / that one: 512 -> 2048 on 128 x 7 x 7 130 / 74, 512 -> 1024 on
-    // 64 x 7 x 7 46 / 43; but 1024 -> 1024 on 32 x 32 x 32 127 / 172, 256 -> 1024 on
-    // 32 x 14 x 14 29 / 42, 256 -> 256 on 24 x 13 x 14 17 / 30).
     const C1WgPlan p = c1_wgrad_plan(B, Cin, Cout, q.P);
     const int64_t n = int64_t(Cin) * Cout;
     if (n > 0x7FFFFFFF || p.steps > 0x7FFFFFFF || p.mt > 65535 || p.nt > 65535) return 0;
-    return n < (int64_t(1) << 19) || int64_t(B) * q.P >= 16384;
+    // Many outputs from few pixels: 2 copies to channel-major rows and one product on 256 x 256
+    // tiles (us, this form / that one: 512 -> 2048 on 128 x 7 x 7 130 / 74, 512 -> 1024 on
+    // 64 x 7 x 7 46 / 43; but 1024 -> 1024 on 32 x 32 x 32 127 / 172).
+    if (n >= (int64_t(1) << 19) && int64_t(B) * q.P < 16384) return 0;
+    return c1_wgrad_us(p, B, Cin, Cout, H, W, q, stride) < 0.88 * c1_wgrad_gemm_us(B, Cin, Cout, H, W, q, stride);
   }
   const int M = op == 1 ? Cin : Cout, K = op == 1 ? Cout : Cin;
   const bool narrow = c1_narrow(M);
   const int64_t gx = int64_t(B) * ceil_div(q.P, narrow ? 128 : 64), gy = ceil_div(M, narrow ? 64 : 128);
-  if (gx > 0x7FFFFFFF || gy > 65535) return 0;
+  if (gx > kMaxGridX || gy > 65535) return 0;
   // A long k on planes whose rows the large GEMM tiles fill and load whole (1024 -> 1024 on
-  // 32 x 32 x 32: 160 / 96 forward, 124 / 74 input gradient; on 14 x 14 planes 55 / 71).
-  if (K >= 1024 && q.P > 256 && q.P % 8 == 0) return 0;
-  // Few workgroups on a long k are a chain of load latencies, which the GEMM's k groups and
-  // splits cut (forward, 2048 -> 512 on 8 x 7 x 7: 41 / 16; input gradient of 256 -> 512 stride
-  // 2 on 8 x 8 x 8: 11.4 / 8.5, on 128 x 8 x 8, 256 workgroups: 16.5 / 17.5).
+  // 32 x 32 x 32: 160 / 96 forward, 124 / 74 input gradient; 1024 -> 2048 on 50 x 16 x 16, 400
+  // tiles, 127 / 90, but input gradient of 256 -> 1024 on 43 x 16 x 16, 43 tiles, 21 / 73).
+  if (K >= 1024 && q.P % 8 == 0 && (q.P > 256 || (q.P == 256 && int64_t(B) * ceil_div(M, 256) >= 200))) return 0;
+  // Few workgroups on a long k (forward, 2048 -> 512 on 8 x 7 x 7: 41 / 16; 2048 -> 2048 on 4 x 14 x 14
+  // 66 / 43; input gradient of 256 -> 512 stride 2 on 8 x 8 x 8: 11.4 / 8.5).
   if (gx * gy < 256 && (op == 0 ? K >= 1024 : stride == 2 && K >= 512)) return 0;
-  return 1;
+  // From 512 workgroups the chains overlap and these kernels win (half the product's time) but for
+  // strided planes of short rows.
+  if (gx * gy >= 512 && (stride == 1 || (op == 0 ? c1_row_breaks(q) < 3 : W >= 16))) return 1;
+  return c1_us(op == 1, gx * gy, B, M, K, Cin, H, W, q, stride) < 0.88 * c1_gemm_us(op == 1, B, M, K, Cin, H, W, q, stride);
 }
 
 int xdna_conv1x1_fwd_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int B, int Cin,
