@@ -39,7 +39,7 @@ struct GArgs {
   uint16_t* out;         // forward: y; dgrad: dx
   float* part;           // wgrad: [nsplit][M][N]
   int B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw, Ho, Wo;
-  int M, N, K, kt_per, nsplit, act;
+  int M, N, K, kt_per, nsplit, act;  // act: 0 none, 1 ReLU
   int x_bytes, w_bytes, dy_bytes;  // operand extents (each under 2^31 bytes)
 };
 
@@ -190,7 +190,9 @@ __device__ inline void gather_a(const GArgs& a, const GRs& rs, int m, int k0, ui
   }
 }
 
-template <int DIR, int TM, bool S1>
+// ReLU a kernel of its own: an activation chosen at run time in the epilogue, whose 16-element chains
+// bound small calls, took 3 us (3 -> 194 3x3 on 2411 x 2 x 2 8.5 -> 11.3).
+template <int DIR, int TM, bool S1, bool RELU>
 __global__ __launch_bounds__(256) void conv_gather_kernel(GArgs a) {
   constexpr int WMW = TM == 32 ? 1 : 2;        // waves along M
   constexpr int WNW = 4 / WMW;                 // waves along N
@@ -293,7 +295,8 @@ __global__ __launch_bounds__(256) void conv_gather_kernel(GArgs a) {
           if (m >= a.M) continue;
           float v = acc[i][j][r];
           if (DIR == kGFwd && a.bias) v += bf16_to_f32(a.bias[m]);
-          o[int64_t(m) * plane] = f32_to_bf16(act_forward(a.act, 0.0f, v));
+          if (RELU && v <= 0.0f) v = 0.0f;  // (a NaN is kept)
+          o[int64_t(m) * plane] = f32_to_bf16(v);
         }
     }
   }
@@ -609,11 +612,11 @@ bool gconv_args(const char* what, GArgs& a, int B, int Cin, int Cout, int H, int
 
 int tile_m(int M) { return M <= 32 ? 32 : M <= 64 ? 64 : 128; }
 
-template <int DIR, bool S1>
+template <int DIR, bool S1, bool RELU = false>
 void launch_gather_s(GArgs& a, dim3 grid, int tm, hipStream_t st) {
-  if (tm == 32) conv_gather_kernel<DIR, 32, S1><<<grid, 256, 0, st>>>(a);
-  else if (tm == 64) conv_gather_kernel<DIR, 64, S1><<<grid, 256, 0, st>>>(a);
-  else conv_gather_kernel<DIR, 128, S1><<<grid, 256, 0, st>>>(a);
+  if (tm == 32) conv_gather_kernel<DIR, 32, S1, RELU><<<grid, 256, 0, st>>>(a);
+  else if (tm == 64) conv_gather_kernel<DIR, 64, S1, RELU><<<grid, 256, 0, st>>>(a);
+  else conv_gather_kernel<DIR, 128, S1, RELU><<<grid, 256, 0, st>>>(a);
 }
 
 template <int DIR>
@@ -622,6 +625,7 @@ int launch_gather(GArgs& a, hipStream_t st) {
   const dim3 grid(unsigned(ceil_div(a.N, kGTN)), unsigned(ceil_div(a.M, tm)), unsigned(a.nsplit));
   // unit strides only change the dgrad gather (no division); one instantiation otherwise
   if (DIR == kGDgrad && a.sh == 1 && a.sw == 1) launch_gather_s<DIR, true>(a, grid, tm, st);
+  else if (DIR == kGFwd && a.act) launch_gather_s<DIR, false, DIR == kGFwd>(a, grid, tm, st);
   else launch_gather_s<DIR, false>(a, grid, tm, st);
   return check_launch("conv gather");
 }
@@ -800,7 +804,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (co < a.Cout) {
         float v = acc[j][r];
         if (a.bias) v += bf16_to_f32(a.bias[co]);
-        o[int64_t(co) * a.Ho * a.Wo] = f32_to_bf16(act_forward(a.act, 0.0f, v));
+        if (a.act & (v <= 0.0f)) v = 0.0f;  // ReLU (a NaN is kept)
+        o[int64_t(co) * a.Ho * a.Wo] = f32_to_bf16(v);
       }
     }
   }

@@ -168,3 +168,28 @@ def test_invalid_shapes(hip):
     assert hip.xdna_conv2d_fwd_bf16(ptr(y), ptr(y), None, ptr(y), 1, 1, 1, 2, 2, 5, 5, 1, 1, 0, 0, stream()) == -1
     assert "kernel larger" in hip.xdna_hip_last_error().decode()
     assert hip.xdna_conv2d_fwd_bf16(ptr(y), ptr(y), None, ptr(y), 1, 1, 1, 2, 2, 1, 1, 0, 1, 0, 0, stream()) == -1
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("case", [(2, 20, 30, 9, 13, 5, 3, 1, 1, 2, 1), (2, 3, 40, 8, 11, 3, 3, 1, 1, 1, 1),
+                                  (2, 24, 3, 8, 11, 5, 5, 1, 1, 2, 2), (2, 3, 70, 17, 15, 7, 7, 2, 2, 3, 3)],
+                         ids=lambda c: "x".join(map(str, c)))
+def test_forward_with_relu_is_relu_of_the_forward(hip, case, variant):
+    """Every forward kernel's ReLU, bit for bit, a NaN kept."""
+    B, Cin, Cout, H, W, KH, KW, sh, sw, ph, pw = case
+    print(f"conv2d relu {case} variant {variant}", flush=True)
+    x, w, b, dy, Ho, Wo = _data(case, sum(case) + 4)
+    x[0, 0, 0, 0] = 0x7FC0
+    xd, wd, bd = dev(x), dev(w), dev(b)
+    plain, relu = dev_zeros((B, Cout, Ho, Wo)), dev_zeros((B, Cout, Ho, Wo))
+    assert hip.xdna_conv2d_set_variant(variant) == 0
+    try:
+        for bias in (None, ptr(bd)):
+            assert hip.xdna_conv2d_fwd_bf16(ptr(xd), ptr(wd), bias, ptr(plain), *case, stream()) == 0
+            assert hip.xdna_conv2d_fwd_act_bf16(ptr(xd), ptr(wd), bias, ptr(relu), *case, 1, stream()) == 0
+            v = host(plain)
+            ref = np.where(oracle.bf16_value(v) <= 0, 0, v)
+            assert np.isnan(oracle.bf16_value(v)).any()
+            np.testing.assert_array_equal(host(relu), ref)
+    finally:
+        assert hip.xdna_conv2d_set_variant(0) == 0
