@@ -407,13 +407,19 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
                            int Cout, int H, int W, int KH, int KW, int sh, int sw, int ph, int pw,
                            void* stream);
 
-/* Kernel selection of xdna_conv2d_fwd_bf16 / xdna_conv2d_dgrad_bf16, for measurements and
- * tests: 0 automatic (default: at stride 1 with few channels on one side, the kernels that put
- * kernel columns beside those channels; else at stride 1 with at most 32 output and at least 16 input
- * channels of the direction, and a padded output width up to 128, the direct form, which stages the
- * input rows of 4 output rows in LDS as a zero-padded grid and reads every tap as a row
- * offset; else the gather GEMM), 1 the gather GEMM only.  No reference counterpart. */
+/* Kernel selection of xdna_conv2d_*, for measurements and tests: 0 automatic (default: at stride 1
+ * with few channels on one side, the kernels that put kernel columns beside those channels, where
+ * they are the faster ones; else at stride 1 with at most 32 output and at least 16 input channels
+ * of the direction, and a padded output width up to 128, the direct form, which stages the input
+ * rows of 4 output rows in LDS as a zero-padded grid and reads every tap as a row offset; else
+ * the gather GEMM), 1 the gather GEMM only, 2 as 0 with the few-channel kernels wherever they
+ * apply.  No reference counterpart. */
 int xdna_conv2d_set_variant(int variant);
+/* Which few-channel kernel takes a stride-1 conv (op 0 forward, 1 input gradient, 2 weight gradient;
+ * bias: whether a bias is added): 1 the few-outputs one, 2 few inputs, 3 weight gradient, 0 none.
+ * op 3: whether the input gradient of a 3x3 / pad-1 layer of few input channels is better off there
+ * than on the packed rows.  -1 for an invalid shape. */
+int xdna_conv2d_few_pick(int op, int B, int Cin, int Cout, int H, int W, int KH, int KW, int ph, int pw, int bias);
 
 /* Kernel selection of xdna_conv3x3_rows_bf16 (and the conv calls built on it), for
  * measurements and tests: 0 automatic (default), 1 the main kernel (128 output channels

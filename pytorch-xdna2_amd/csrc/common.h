@@ -144,6 +144,9 @@ struct __attribute__((packed, aligned(2))) Pix8 {
   uint32_t v[4];
 };
 
+// Most workgroups of 256 threads along a grid's x (its threads stay under 2^32).
+constexpr int64_t kMaxGridX256 = (int64_t(1) << 24) - 1;
+
 // n / d for n * d < 2^32 and d > 1, with m = 0xFFFFFFFF / d + 1: one multiply instead of
 // the ~20 instructions of a division by a run-time value.
 __device__ inline int fast_div(int n, uint32_t m) { return int(__umulhi(uint32_t(n), m)); }

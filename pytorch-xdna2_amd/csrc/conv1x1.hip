@@ -346,8 +346,6 @@ __global__ __launch_bounds__(256) void conv1x1_wgrad_reduce_kernel(const float* 
   gw[e] = f32_to_bf16(s);
 }
 
-constexpr int64_t kMaxGridX = (int64_t(1) << 24) - 1;  // workgroups of 256 threads: a grid side under 2^32 threads
-
 struct C1Geom {
   int Ho, Wo, P;
 };
@@ -387,7 +385,7 @@ int c1_launch(const char* who, bool dx, const uint16_t* x, const uint16_t* w, co
   const bool narrow = c1_narrow(g.M);
   g.tpi = int(ceil_div(q.P, narrow ? 128 : 64));
   const int64_t gx = int64_t(B) * g.tpi, gy = ceil_div(g.M, narrow ? 64 : 128);
-  if (gx > kMaxGridX || gy > 65535) {
+  if (gx > kMaxGridX256 || gy > 65535) {
     set_error(std::string(who) + ": grid too large");
     return -1;
   }
@@ -518,7 +516,7 @@ int xdna_conv1x1_pick(int op, int B, int Cin, int Cout, int H, int W, int stride
   const int M = op == 1 ? Cin : Cout, K = op == 1 ? Cout : Cin;
   const bool narrow = c1_narrow(M);
   const int64_t gx = int64_t(B) * ceil_div(q.P, narrow ? 128 : 64), gy = ceil_div(M, narrow ? 64 : 128);
-  if (gx > kMaxGridX || gy > 65535) return 0;
+  if (gx > kMaxGridX256 || gy > 65535) return 0;
   // A long k on planes whose rows the large GEMM tiles fill and load whole (1024 -> 1024 on
   // 32 x 32 x 32: 160 / 96 forward, 124 / 74 input gradient; 1024 -> 2048 on 50 x 16 x 16, 400
   // tiles, 127 / 90, but input gradient of 256 -> 1024 on 43 x 16 x 16, 43 tiles, 21 / 73).

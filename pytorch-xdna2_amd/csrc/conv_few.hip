@@ -17,8 +17,8 @@
 // 40 x 36 x 36 pixels, 9x9, us in a graph on an MI355X, against the direct, gather and
 // sliding-window kernels of conv_gather.hip: 32 -> 3 forward 27.7 -> 11.7, input gradient
 // 21.4 -> 8.2, weight and bias gradients 51.0 -> 20.8; 3 -> 32 23.1 -> 8.5, 25.9 -> 11.4,
-// 33.0 -> 17.8.  They take every shape they fit: 3x3 3 -> 64 at 128 x 64 x 64 44 -> 30,
-// 82 -> 51, 153 -> 76.
+// 33.0 -> 17.8; 3x3 3 -> 64 at 128 x 64 x 64 44 -> 30, 82 -> 51, 153 -> 76.  The rules beside the plans
+// say where the general kernels stay ahead.
 #include "conv_few.h"
 
 #include "common.h"
@@ -36,7 +36,9 @@ constexpr int kFewWeights = 16;           // weight loads in flight per thread
 
 // Every kernel below may use up to a CU's LDS.
 bool raise_lds(const void* fn) {
-  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(kFewLdsMax)) == hipSuccess;
+  const bool ok = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, int(kFewLdsMax)) == hipSuccess;
+  if (!ok) (void)hipGetLastError();  // (the general kernels take the call)
+  return ok;
 }
 
 // Calls put(row, chan, tap, value) for `rows` x `chans` x `taps` weights from row0, chan0 on;
@@ -222,9 +224,10 @@ size_t few_out_lds(const FewOutArgs& a) {
   return std::max(size_t(a.xpos + a.KH * 32) * kFewPitch * 2, size_t(a.Cout) * a.KW * (a.nb * 32 + 1) * 4);
 }
 
-int run_few_out(FewOutArgs a, hipStream_t st) {
+// Fills in the geometry; false where the kernel does not apply or (unless `any`) loses.
+bool few_out_plan(FewOutArgs& a, bool any) {
   // at least 8 input channels (below, the 32-channel chunk is mostly padding)
-  if (a.Cout * a.KW > 32 || a.Cin < 8 || a.W < 4) return 1;
+  if (a.KH > 16 || a.KH < 1 || a.KW < 1 || a.Cout * a.KW > 32 || a.Cin < 8 || a.W < 4) return false;
   a.Wp = a.Wo + a.KW - 1;
   // rows per workgroup: the fewest rounds of workgroups (two per CU in half its LDS) times
   // rows staged in each
@@ -243,12 +246,21 @@ int run_few_out(FewOutArgs a, hipStream_t st) {
       cost = c;
     }
   }
-  if (!best) return 1;
+  if (!best) return false;
   a.R = best;
   a.nb = int(ceil_div(int64_t(a.R) * a.Wp, 32));
   a.xpos = a.nb * 32 + (a.KH - 1) * a.Wp;
   a.rtiles = int(ceil_div(a.Ho, a.R));
-  if (int64_t(a.B) * a.rtiles > 0x7fffffff) return 1;
+  // A batch of planes of up to 64 pixels over more than two workgroups per CU: the gather's tiles
+  // run over the images, and up to four of its k-tiles are no chain (9 -> 3 on 2032 x 3 x 3 15.8
+  // against 8.0 us; longer ones gain all the same: 16 -> 1 9x9 on 657 x 4 x 4 8.5 against 29.9).
+  if (!any && int64_t(a.Ho) * a.Wo <= 64 && int64_t(a.B) * a.rtiles > 512 && int64_t(a.Cin) * a.KH * a.KW <= 128)
+    return false;
+  return int64_t(a.B) * a.rtiles <= kMaxGridX256;
+}
+
+int run_few_out(FewOutArgs a, bool any, hipStream_t st) {
+  if (!few_out_plan(a, any)) return 1;
   static const bool ok = raise_lds(reinterpret_cast<const void*>(&few_out_kernel<1>)) &&
                          raise_lds(reinterpret_cast<const void*>(&few_out_kernel<2>)) &&
                          raise_lds(reinterpret_cast<const void*>(&few_out_kernel<3>)) &&
@@ -416,45 +428,78 @@ __global__ __launch_bounds__(256) void few_in_kernel(FewInArgs a) {
   }
 }
 
+// The tile of a conv of KW columns: 32 mt channels x 128 np pixels; np 0 where the kernel does
+// not apply or loses.
+struct FewInPlan {
+  int mt = 0, np = 0;
+  size_t lds = 0;
+};
+
+// Where the kernel is the better one, in `wgs` tiles of 64 channels x 128 pixels (us, this one /
+// the gather): planes that fill less than half of a tile only while two workgroups per CU hold
+// them all (3 -> 102 3x3 on 1859 x 4 x 4 45 / 9.2, 1 -> 254 7x7 on 445 x 4 x 4, 46 / 11.3; on up to
+// 512 workgroups 0.4-0.9 of its time).  With a bias, which the gather adds element by element,
+// everything else (0.3-0.9).  Without one, a lone input channel leaves three of four channel slots
+// empty, so not 5 columns (25 taps are one k-tile of the gather: 1.0-1.5 of its time) nor many
+// workgroups (1 -> 228 9x9 on 73 x 63 x 9 41 / 23); and taps that fill one k-tile of the gather (3x3
+// of 3 channels) leave nothing to gain but the wide stores of more than 64 channels on a few
+// hundred workgroups (0.93; 1.09 past 1024) or of many pixels on fewer channels.
+bool few_in_pays(const FewInArgs& a, int KW) {
+  const int64_t px = int64_t(a.Ho) * a.Wo, wgs = a.B * ceil_div(px, 128) * ceil_div(a.Cout, 64);
+  if (px <= 64 && wgs > 512) return false;
+  if (a.bias) return true;
+  if (a.Cin == 1 && (KW == 5 || wgs > 1024)) return false;
+  if (a.Cin * a.KH * KW <= 32) return a.Cout > 64 ? wgs <= 1024 : wgs > 512;
+  return true;
+}
+
+FewInPlan few_in_plan(const FewInArgs& a, int KW, bool any) {
+  FewInPlan p;
+  if (a.KH > 16 || a.KH < 1 || (KW != 3 && KW != 5 && KW != 7 && KW != 9) || a.Cin > 4 || ceil_div(a.Cout, 32) > 65535 ||
+      !(any || few_in_pays(a, KW)))
+    return p;
+  p.mt = a.Cout > 32 ? 2 : 1;
+  const int64_t px = int64_t(a.Ho) * a.Wo;
+  // 256 pixels per workgroup where that still gives two workgroups per CU (a workgroup's
+  // weights and halo rows are staged once per tile), else 128.
+  for (int np = a.B * ceil_div(px, 256) * ceil_div(a.Cout, 64) >= 512 ? 2 : 1; np > 0 && !p.np; --np) {
+    const int pix = 128 * np;
+    // the most input rows `pix` consecutive pixels read
+    const int rows = std::min((pix - 2) / a.Wo + 2, a.Ho) + a.KH - 1;
+    p.lds = std::max(size_t(a.KH) * ((KW + 3) / 4) * 2 * 32 * p.mt * 16 +
+                         size_t(int64_t(rows) * (a.Wo + KW - 1) + kFewInPad) * 8,
+                     size_t(32 * p.mt) * (pix + 8) * 2);
+    if (p.lds <= kFewLdsMax && a.B * ceil_div(px, pix) <= kMaxGridX256) p.np = np;
+  }
+  return p;
+}
+
 template <int KW, int MT, int NP>
-int launch_few_in_np(FewInArgs a, hipStream_t st) {
+int launch_few_in_np(FewInArgs a, size_t lds, hipStream_t st) {
   static const bool ok = raise_lds(reinterpret_cast<const void*>(&few_in_kernel<KW, MT, NP>));
   if (!ok) return 1;
-  constexpr int kPix = 128 * NP;
-  a.tiles = int(ceil_div(int64_t(a.Ho) * a.Wo, kPix));
-  // the most input rows kPix consecutive pixels read
-  const int rows = std::min((kPix - 2) / a.Wo + 2, a.Ho) + a.KH - 1;
-  const size_t lds = std::max(size_t(a.KH) * ((KW + 3) / 4) * 2 * 32 * MT * 16 + size_t(rows * a.Wp + kFewInPad) * 8,
-                              size_t(32 * MT) * (kPix + 8) * 2);
-  if (lds > kFewLdsMax || int64_t(a.B) * a.tiles > 0x7fffffff) return 1;
+  a.tiles = int(ceil_div(int64_t(a.Ho) * a.Wo, 128 * NP));
   const dim3 grid(unsigned(a.B * a.tiles), unsigned(ceil_div(a.Cout, 32 * MT)));
   few_in_kernel<KW, MT, NP><<<grid, 256, lds, st>>>(a);
   return check_launch("conv few inputs");
 }
 
-// 256 pixels per workgroup where that still gives two workgroups per CU (a workgroup's
-// weights and halo rows are staged once per tile), else 128.
 template <int KW>
-int launch_few_in(const FewInArgs& a, hipStream_t st) {
-  const bool large = a.B * ceil_div(int64_t(a.Ho) * a.Wo, 256) * ceil_div(a.Cout, 64) >= 512;
-  if (a.Cout > 32) {
-    const int rc = large ? launch_few_in_np<KW, 2, 2>(a, st) : 1;
-    return rc <= 0 ? rc : launch_few_in_np<KW, 2, 1>(a, st);
-  }
-  const int rc = large ? launch_few_in_np<KW, 1, 2>(a, st) : 1;
-  return rc <= 0 ? rc : launch_few_in_np<KW, 1, 1>(a, st);
+int launch_few_in(const FewInArgs& a, const FewInPlan& p, hipStream_t st) {
+  if (p.mt == 2) return p.np == 2 ? launch_few_in_np<KW, 2, 2>(a, p.lds, st) : launch_few_in_np<KW, 2, 1>(a, p.lds, st);
+  return p.np == 2 ? launch_few_in_np<KW, 1, 2>(a, p.lds, st) : launch_few_in_np<KW, 1, 1>(a, p.lds, st);
 }
 
-int run_few_in(FewInArgs a, int KW, hipStream_t st) {
-  if (a.Cin > 4 || ceil_div(a.Cout, 32) > 65535) return 1;
+int run_few_in(FewInArgs a, int KW, bool any, hipStream_t st) {
+  const FewInPlan p = few_in_plan(a, KW, any);
+  if (!p.np) return 1;
   a.Wp = a.Wo + KW - 1;
   switch (KW) {
-    case 3: return launch_few_in<3>(a, st);
-    case 5: return launch_few_in<5>(a, st);
-    case 7: return launch_few_in<7>(a, st);
-    case 9: return launch_few_in<9>(a, st);
+    case 3: return launch_few_in<3>(a, p, st);
+    case 5: return launch_few_in<5>(a, p, st);
+    case 7: return launch_few_in<7>(a, p, st);
+    default: return launch_few_in<9>(a, p, st);
   }
-  return 1;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -678,27 +723,13 @@ __global__ __launch_bounds__(256) void few_wgrad_reduce_kernel(const float* __re
   gw[(at * a.KH + ky) * a.KW + kx] = f32_to_bf16(s);
 }
 
-}  // namespace
-
-int conv_few_fwd(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* out, int B, int Cin, int Cout,
-                 int H, int W, int KH, int KW, int ph, int pw, int flip, int act, hipStream_t st) {
-  const int Ho = H + 2 * ph - KH + 1, Wo = W + 2 * pw - KW + 1;
-  if (KH > 16 || KH < 1 || KW < 1) return 1;
-  FewOutArgs o{x, w, bias, out, B, Cin, Cout, H, W, KH, KW, ph, pw, Ho, Wo, flip, act, 0, 0, 0, 0, 0};
-  const int rc = run_few_out(o, st);
-  if (rc <= 0) return rc;
-  FewInArgs i{x, w, bias, out, B, Cin, Cout, H, W, KH, ph, pw, Ho, Wo, flip, act, 0, 0};
-  return run_few_in(i, KW, st);
-}
-
-int conv_few_wgrad(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t* gb, int B, int Cin, int Cout, int H,
-                   int W, int KH, int KW, int ph, int pw, hipStream_t st) {
-  FewWgArgs a{};
+// The weight gradient's geometry (operands and outputs left out); 0 LDS bytes where the kernel
+// does not apply or (unless `any`) loses.
+size_t few_wgrad_plan(FewWgArgs& a, int B, int Cin, int Cout, int H, int W, int KH, int KW, int ph, int pw, bool bias,
+                      bool any) {
   a.Ho = H + 2 * ph - KH + 1;
   a.Wo = W + 2 * pw - KW + 1;
   const bool few_dy = Cout <= Cin;
-  a.wide = few_dy ? x : dy;
-  a.few = few_dy ? dy : x;
   a.Cw = few_dy ? Cin : Cout;
   a.Cf = few_dy ? Cout : Cin;
   a.Hw = few_dy ? H : a.Ho;
@@ -708,13 +739,21 @@ int conv_few_wgrad(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t
   a.KH = KH; a.KW = KW; a.ph = ph; a.pw = pw;
   a.M = a.Cf * KW;
   // (pw <= KW: a shifted row then stays within the zeros kept around it)
-  if (pw > KW || a.Cf > 4 || a.Cw < 8 || KH > 8 * kFewMaxKy || KW < 3 || a.M > 32 || a.Ww < 4) return 1;
+  if (pw > KW || a.Cf > 4 || a.Cw < 8 || KH > 8 * kFewMaxKy || KH < 1 || KW < 3 || a.M > 32 || a.Ww < 4) return 0;
+  // Few inputs: a tile is one image's, so planes of up to 64 pixels (3 -> 254 5x5 on 1266 x 4 x 4 94
+  // against the general kernels' 29 us; from 7x7 on up to 25) and up to 64 channels on a few thousand
+  // pixels, one tile's latency against splits over the chip (3 -> 22 9x9 on 4 x 45 x 22 14.8 / 10.3),
+  // stay there.  A bias, whose gradient is a pass of its own there, draws the two level; it has no
+  // say, so that the weight gradient has the same bits with and without.  Few outputs gain
+  // throughout (0.2-0.9).
+  const int64_t px = int64_t(a.Ho) * a.Wo;
+  if (!any && !few_dy && (px <= (KH * KW >= 49 ? 25 : 64) || (Cout <= 64 && B * px < 8000))) return 0;
   a.Wq = (a.Ww + 7) & ~7;
   a.wblks = int(ceil_div(a.Cw, 32));
   const int64_t total = int64_t(a.wblks) * KH * a.M * 32 + Cout;
-  if (total > (1 << 24) || a.wblks > 65535) return 1;
+  if (total > (1 << 24) || a.wblks > 65535) return 0;
   a.total = int(total);
-  a.bias = gb != nullptr;
+  a.bias = bias;
   auto geometry = [&](int R) {
     a.R = R;
     a.wrows = few_dy ? R + KH - 1 : R;
@@ -737,11 +776,49 @@ int conv_few_wgrad(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t
       cost = c;
     }
   }
-  if (!best) return 1;
+  if (!best) return 0;
   const size_t lds = geometry(best);
   a.tpi = int(ceil_div(a.Ho, a.R));
-  if (int64_t(B) * a.tpi > 0x7fffffff) return 1;
+  if (int64_t(B) * a.tpi > 0x7fffffff) return 0;
   a.ntiles = B * a.tpi;
+  return lds;
+}
+
+FewOutArgs few_out_args(int B, int Cin, int Cout, int H, int W, int KH, int KW, int ph, int pw) {
+  FewOutArgs a{};
+  a.B = B; a.Cin = Cin; a.Cout = Cout; a.H = H; a.W = W; a.KH = KH; a.KW = KW; a.ph = ph; a.pw = pw;
+  a.Ho = H + 2 * ph - KH + 1;
+  a.Wo = W + 2 * pw - KW + 1;
+  return a;
+}
+
+FewInArgs few_in_args(const FewOutArgs& o) {
+  FewInArgs a{};
+  a.x = o.x; a.w = o.w; a.bias = o.bias; a.out = o.out;
+  a.B = o.B; a.Cin = o.Cin; a.Cout = o.Cout; a.H = o.H; a.W = o.W; a.KH = o.KH; a.ph = o.ph; a.pw = o.pw;
+  a.Ho = o.Ho; a.Wo = o.Wo; a.flip = o.flip; a.act = o.act;
+  return a;
+}
+
+}  // namespace
+
+int conv_few_fwd(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* out, int B, int Cin, int Cout,
+                 int H, int W, int KH, int KW, int ph, int pw, int flip, int act, bool any,
+                 hipStream_t st) {
+  FewOutArgs a = few_out_args(B, Cin, Cout, H, W, KH, KW, ph, pw);
+  a.x = x; a.w = w; a.bias = bias; a.out = out; a.flip = flip; a.act = act;
+  const int rc = run_few_out(a, any, st);
+  return rc <= 0 ? rc : run_few_in(few_in_args(a), KW, any, st);
+}
+
+int conv_few_wgrad(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t* gb, int B, int Cin, int Cout, int H,
+                   int W, int KH, int KW, int ph, int pw, bool any, hipStream_t st) {
+  FewWgArgs a{};
+  const size_t lds = few_wgrad_plan(a, B, Cin, Cout, H, W, KH, KW, ph, pw, gb != nullptr, any);
+  if (!lds) return 1;
+  const bool few_dy = Cout <= Cin;
+  a.wide = few_dy ? x : dy;
+  a.few = few_dy ? dy : x;
   static const bool ok = raise_lds(reinterpret_cast<const void*>(&few_wgrad_kernel<true>)) &&
                          raise_lds(reinterpret_cast<const void*>(&few_wgrad_kernel<false>));
   if (!ok) return 1;
@@ -755,6 +832,22 @@ int conv_few_wgrad(const uint16_t* x, const uint16_t* dy, uint16_t* gw, uint16_t
   few_wgrad_reduce_kernel<<<unsigned(ceil_div(n, 32)), 256, 0, st>>>(a.part, gw, gb, nwg, a, few_dy ? 1 : 0, n);
   xdna_hip_cache_free(a.part);  // stream-ordered reuse: the next user of the block runs after the reduce
   return check_launch("conv few-channel weight gradient");
+}
+
+int conv_few_pick(int op, int B, int Cin, int Cout, int H, int W, int KH, int KW, int ph, int pw, bool bias,
+                  bool any) {
+  if (op == 2) {
+    FewWgArgs a{};
+    return few_wgrad_plan(a, B, Cin, Cout, H, W, KH, KW, ph, pw, bias, any) ? 3 : 0;
+  }
+  // (the input gradient as a forward conv of dy)
+  static const uint16_t one = 0;
+  const bool dx = op == 1;
+  if (dx && (ph > KH - 1 || pw > KW - 1)) return 0;
+  FewOutArgs a = dx ? few_out_args(B, Cout, Cin, H + 2 * ph - KH + 1, W + 2 * pw - KW + 1, KH, KW, KH - 1 - ph, KW - 1 - pw)
+                    : few_out_args(B, Cin, Cout, H, W, KH, KW, ph, pw);
+  a.bias = bias && !dx ? &one : nullptr;
+  return few_out_plan(a, any) ? 1 : few_in_plan(few_in_args(a), KW, any).np ? 2 : 0;
 }
 
 }  // namespace xdna

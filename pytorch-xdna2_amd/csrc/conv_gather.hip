@@ -840,7 +840,7 @@ bool direct_args(DArgs& d, int B, int Cin, int Cout, int H, int W, int KH, int K
 
 size_t direct_lds(const DArgs& d) { return size_t(d.xpos + d.wv * 256 / 4) * kDPitch * 2; }
 
-std::atomic<int> g_conv2d_variant{0};  // 0 automatic, 1 gather GEMM only
+std::atomic<int> g_conv2d_variant{0};  // 0 automatic, 1 gather GEMM only, 2 few-channel kernels wherever they apply
 
 // Runs the direct form (weights prepared into the cache allocator) or returns 1 when it
 // does not apply.
@@ -928,8 +928,9 @@ int xdna_conv2d_fwd_act_bf16(const uint16_t* x, const uint16_t* w, const uint16_
   a.kt_per = int(ceil_div(a.K, kGTK));
   if (!admit_launch("xdna_conv2d_fwd_bf16")) return -1;
   if (sh == 1 && sw == 1) {
-    if (g_conv2d_variant.load() == 0) {
-      const int rc = conv_few_fwd(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, ph, pw, 0, act, as_stream(stream));
+    if (const int v = g_conv2d_variant.load(); v != 1) {
+      const int rc =
+          conv_few_fwd(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, ph, pw, 0, act, v == 2, as_stream(stream));
       if (rc <= 0) return rc;
     }
     const int rc = run_direct(x, w, bias, y, B, Cin, Cout, H, W, KH, KW, ph, pw, 0, act, as_stream(stream));
@@ -950,9 +951,9 @@ int xdna_conv2d_dgrad_bf16(const uint16_t* dy, const uint16_t* w, uint16_t* dx, 
   if (sh == 1 && sw == 1 && ph <= KH - 1 && pw <= KW - 1) {
     // at stride 1 the input gradient is the forward conv of dy with the flipped,
     // transposed weights and padding K - 1 - p, which gives back H x W
-    if (g_conv2d_variant.load() == 0) {
+    if (const int v = g_conv2d_variant.load(); v != 1) {
       const int rc = conv_few_fwd(dy, w, nullptr, dx, B, Cout, Cin, a.Ho, a.Wo, KH, KW, KH - 1 - ph, KW - 1 - pw, 1, 0,
-                                  as_stream(stream));
+                                  v == 2, as_stream(stream));
       if (rc <= 0) return rc;
     }
     const int rc = run_direct(dy, w, nullptr, dx, B, Cout, Cin, a.Ho, a.Wo, KH, KW, KH - 1 - ph, KW - 1 - pw, 1, 0,
@@ -970,8 +971,8 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
   a.x = x; a.dy = dy;
   hipStream_t st = as_stream(stream);
   if (!admit_launch("xdna_conv2d_wgrad_bf16")) return -1;
-  if (sh == 1 && sw == 1 && g_conv2d_variant.load() == 0) {
-    const int rc = conv_few_wgrad(x, dy, gw, gb, B, Cin, Cout, H, W, KH, KW, ph, pw, st);
+  if (const int v = g_conv2d_variant.load(); sh == 1 && sw == 1 && v != 1) {
+    const int rc = conv_few_wgrad(x, dy, gw, gb, B, Cin, Cout, H, W, KH, KW, ph, pw, v == 2, st);
     if (rc <= 0) return rc;
   }
   FsArgs fs{};
@@ -1046,9 +1047,31 @@ int xdna_conv2d_wgrad_bf16(const uint16_t* x, const uint16_t* dy, uint16_t* gw, 
   return 0;
 }
 
+int xdna_conv2d_few_pick(int op, int B, int Cin, int Cout, int H, int W, int KH, int KW, int ph, int pw, int bias) {
+  if (op < 0 || op > 3) {
+    set_error("xdna_conv2d_few_pick: invalid op");
+    return -1;
+  }
+  GArgs a{};
+  if (!gconv_args("xdna_conv2d_few_pick", a, B, Cin, Cout, H, W, KH, KW, 1, 1, ph, pw)) return -1;
+  const int v = g_conv2d_variant.load();
+  if (v == 1) return 0;
+  if (op < 3) return conv_few_pick(op, B, Cin, Cout, H, W, KH, KW, ph, pw, bias != 0, v == 2);
+  // Against the pack and the rows conv: up to 8 output channels leave the chunks empty, and planes
+  // past 256 columns go in strips.  A chunk of 32 channels is a round of this kernel's chain, so from
+  // 64 channels on only where the pixels hide it: us, this one / those, 3 <- 163 on 1 x 23 x 30 17.5 / 11, 1 <- 416 on
+  // 74 x 8 x 8 38 / 21, but 1 <- 289 on 92 x 34 x 18 24 / 57, 3 <- 233 on 64 x 40 x 40 0.55 of the time.  Nor for
+  // batches of planes of up to 64 pixels, one workgroup each (3 <- 57 on 733 x 4 x 4 13.6 -> 19.6).
+  const int64_t px = int64_t(H) * W;
+  if (KH != 3 || KW != 3 || ph != 1 || pw != 1 || Cout < 8 || W > 256 || conv_few_pick(1, B, Cin, Cout, H, W, 3, 3, 1, 1, false, v == 2) != 1)
+    return 0;
+  if (v == 2 || Cout <= 32) return 1;
+  return !(px <= 64 && B > 512) && (Cout <= 64 || B * px >= 75 * int64_t(Cout));
+}
+
 int xdna_conv2d_set_variant(int variant) {
-  if (variant < 0 || variant > 1) {
-    set_error("xdna_conv2d_set_variant: variant must be 0 or 1");
+  if (variant < 0 || variant > 2) {
+    set_error("xdna_conv2d_set_variant: variant must be 0, 1 or 2");
     return -1;
   }
   g_conv2d_variant.store(variant);

@@ -873,8 +873,9 @@ bool gconv_fits_3x3(const at::Tensor& x, const at::Tensor& w) {
   return pixels > 0 && pixels * std::max(x.size(1), w.size(0)) < (int64_t(1) << 30);
 }
 bool few_input_dx(const at::Tensor& x, const at::Tensor& w) {
-  return g_gconv_mode.load() == 2 && !g_bfp16_emul.load() && w.size(0) >= 8 && x.size(3) >= 4 && x.size(3) <= 256 &&
-         gconv_fits_3x3(x, w);
+  return g_gconv_mode.load() == 2 && !g_bfp16_emul.load() && gconv_fits_3x3(x, w) &&
+         xdna_conv2d_few_pick(3, int(x.size(0)), int(x.size(1)), int(w.size(0)), int(x.size(2)), int(x.size(3)), 3, 3, 1, 1,
+                              0) == 1;
 }
 bool gconv_auto_fwd(int cin, int cout, int sh, int sw) {
   return gconv_auto(cout, sh, sw) || (cout <= 32 && cin >= 16 && sh == 1 && sw == 1);

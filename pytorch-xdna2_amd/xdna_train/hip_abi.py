@@ -95,6 +95,7 @@ SIGNATURES = {
     "xdna_upsample_nearest2x_bf16": (I, [P, P, L, I, I, P]),
     "xdna_conv2d_fwd_act_bf16": (I, [P, P, P, P] + [I] * 12 + [P]),
     "xdna_conv2d_set_variant": (I, [I]),
+    "xdna_conv2d_few_pick": (I, [I] * 11),
     "xdna_subsample2_bf16": (I, [P, P, L, I, I, P]),
     "xdna_conv3x3_prepare_weights_both_bf16": (I, [P, P, P, I, I, P]),
     "xdna_conv3x3_wgrad_rows_workspace_bytes": (Z, [I, I, I, I, I, I]),

@@ -27,3 +27,40 @@ CONV1X1 = [
 def test_conv1x1_takes_the_faster_form(shape, here, product):
     want = 1 if here is None or here < 1.05 * product else 0
     assert hip_abi.load().xdna_conv1x1_pick(*shape) == want
+
+
+# op (0 forward, 1 input gradient, 2 weight gradient, 3 the 3x3 input gradient against the packed-rows
+# conv), B, Cin, Cout, H, W, K, padding, bias: us of the few-channel kernel, us of the other
+FEW = [
+    # batches of planes that fill no tile; one input channel; taps of one k-tile; long chains of chunks
+    ((0, 1859, 3, 102, 4, 4, 3, 1, 0), 45, 9.2), ((0, 445, 1, 254, 4, 4, 7, 3, 0), 46, 11.3),
+    ((0, 2091, 4, 336, 8, 8, 3, 0, 1), 171, 60), ((1, 430, 194, 1, 2, 2, 9, 4, 0), 65, 12.8),
+    ((1, 73, 228, 1, 63, 9, 9, 4, 0), 40.5, 23.0), ((0, 32, 1, 52, 102, 107, 5, 2, 0), 34.5, 23.3),
+    ((0, 84, 3, 238, 34, 31, 3, 1, 0), 32.4, 24.2), ((0, 3, 1, 9, 24, 109, 3, 0, 0), 5.7, 4.6),
+    ((0, 2032, 9, 3, 5, 5, 3, 0, 0), 15.8, 8.0), ((2, 1266, 3, 254, 4, 4, 5, 2, 0), 94, 29),
+    ((2, 4, 3, 22, 45, 22, 9, 4, 0), 14.8, 10.3), ((2, 773, 1, 127, 5, 5, 3, 1, 1), 51.7, 34.8),
+    ((3, 1, 3, 163, 23, 30, 3, 1, 0), 17.5, 11.0), ((3, 74, 1, 416, 8, 8, 3, 1, 0), 38, 21),
+    ((3, 733, 3, 57, 4, 4, 3, 1, 0), 19.6, 13.6), ((3, 1, 3, 233, 10, 87, 3, 1, 0), 26.6, 13.9),
+    # the layers they were made for
+    ((0, 40, 3, 32, 36, 36, 9, 4, 1), 8.5, 23.1), ((1, 40, 3, 32, 36, 36, 9, 4, 0), 11.4, 25.9),
+    ((2, 40, 3, 32, 36, 36, 9, 4, 1), 17.8, 33.0), ((0, 40, 32, 3, 36, 36, 9, 4, 1), 11.7, 27.7),
+    ((1, 40, 32, 3, 36, 36, 9, 4, 0), 8.2, 21.4), ((2, 40, 32, 3, 36, 36, 9, 4, 1), 20.8, 51.0),
+    ((0, 128, 3, 64, 64, 64, 3, 1, 0), 30, 44), ((3, 128, 3, 64, 64, 64, 3, 1, 0), 51, 82),
+    ((2, 128, 3, 64, 64, 64, 3, 1, 0), 76, 153), ((0, 2233, 335, 3, 5, 5, 7, 3, 0), 190, 1180),
+    ((0, 40, 3, 138, 10, 71, 3, 1, 1), 8.8, 18.0), ((3, 40, 3, 64, 36, 36, 3, 1, 0), 9.8, 13.3),
+]
+
+
+@pytest.mark.parametrize("shape,here,other", FEW, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_few_channel_convs_take_the_faster_form(shape, here, other):
+    op, B, cin, cout, H, W, K, p, bias = shape
+    got = hip_abi.load().xdna_conv2d_few_pick(op, B, cin, cout, H, W, K, K, p, p, bias)
+    assert (got > 0) == (here < other)
+
+
+def test_grids_past_the_launch_limit_stay_off_the_few_channel_kernels():
+    """A workgroup per image of 256 threads: 2^24 of them are more threads than a launch takes."""
+    lib = hip_abi.load()
+    pick = lambda op, *a: lib.xdna_conv2d_few_pick(op, *a, 3, 3, 1, 1, 1)  # noqa: E731
+    assert pick(0, 1 << 24, 8, 3, 1, 4) == 0 and pick(0, 1 << 24, 3, 8, 1, 4) == 0 and pick(1, 1 << 24, 3, 8, 1, 4) == 0
+    assert lib.xdna_conv1x1_pick(0, 1 << 24, 8, 8, 1, 4, 1) == 0

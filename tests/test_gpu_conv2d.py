@@ -134,6 +134,33 @@ def test_few_channels(hip, case):
     check_bf16(host(gb), ref_b, what=f"bias grad {case}")
 
 
+# which kernel applies to each of those, forward, input gradient and weight gradient (1 few outputs,
+# 2 few inputs, 3 the weight gradient's, 0 none: paddings past the kernel), and two layers of more
+# wide channels than a tile
+FEW_ROUTES = [(1, 2, 3)] * 3 + [(2, 1, 3)] * 4 + [(1, 2, 3)] * 2 + [(2, 1, 3), (1, 2, 3), (2, 1, 3), (1, 0, 3), (2, 0, 0), (1, 0, 0)]
+FEW_APPLY = list(zip(FEW, FEW_ROUTES)) + [((1, 300, 3, 6, 9, 3, 3, 1, 1, 1, 1), (1, 2, 3)),
+                                          ((1, 3, 300, 6, 9, 3, 3, 1, 1, 1, 1), (2, 1, 3))]
+
+
+@pytest.fixture
+def few_everywhere(hip):
+    assert hip.xdna_conv2d_set_variant(2) == 0
+    yield
+    assert hip.xdna_conv2d_set_variant(0) == 0
+
+
+@pytest.mark.parametrize("case,routes", FEW_APPLY, ids=lambda c: "x".join(map(str, c)))
+def test_few_channels_wherever_they_apply(hip, case, routes, few_everywhere):
+    """The few-channel kernels at the edges of their tiles, whichever kernels the choice would take."""
+    assert tuple(hip.xdna_conv2d_few_pick(op, *case[:7], *case[9:], 1) for op in range(3)) == routes
+    test_few_channels(hip, case)
+
+
+@pytest.mark.parametrize("cin,cout", [(12, 3), (3, 12)])
+def test_few_channels_keep_infinities_wherever_they_apply(hip, cin, cout, few_everywhere):
+    test_few_channels_keep_infinities_in_their_pairs(hip, cin, cout)
+
+
 @pytest.mark.parametrize("cin,cout", [(12, 3), (3, 12)])
 def test_few_channels_keep_infinities_in_their_pairs(hip, cin, cout):
     """An infinity in x reaches the outputs whose window holds it and the weight gradients of
@@ -170,7 +197,7 @@ def test_invalid_shapes(hip):
     assert hip.xdna_conv2d_fwd_bf16(ptr(y), ptr(y), None, ptr(y), 1, 1, 1, 2, 2, 1, 1, 0, 1, 0, 0, stream()) == -1
 
 
-@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("variant", [0, 1, 2])
 @pytest.mark.parametrize("case", [(2, 20, 30, 9, 13, 5, 3, 1, 1, 2, 1), (2, 3, 40, 8, 11, 3, 3, 1, 1, 1, 1),
                                   (2, 24, 3, 8, 11, 5, 5, 1, 1, 2, 2), (2, 3, 70, 17, 15, 7, 7, 2, 2, 3, 3)],
                          ids=lambda c: "x".join(map(str, c)))
