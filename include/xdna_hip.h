@@ -373,7 +373,8 @@ int xdna_conv3x3_px_bf16(int form, const uint16_t* xp, const uint16_t* wt, const
 
 /* Whether these kernels are the better choice (and take the operands): op 0 stride-1 conv, 1
  * stride-2 forward, 2 stride-2 input gradient, 3 stride-1 weight gradient, 4 stride-2 weight
- * gradient.  0 where a kernel of the rows or weight-gradient forms is forced. */
+ * gradient, against the kernels on the same packed rows; 5 / 6 as 0 / 1 with the pack, against
+ * xdna_conv3x3_nchw_act_bf16.  0 where a kernel of the rows or weight-gradient forms is forced. */
 int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int layout);
 /* Their weight gradient (form 0 or 1; + bias gradient when gb is not null) from the packed rows
  * of x (H x W) and of the conv's output gradient; the pixel reduction is split over workgroups

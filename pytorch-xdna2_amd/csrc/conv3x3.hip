@@ -3535,19 +3535,35 @@ int xdna_conv3x3_px_bf16(int form, const uint16_t* xp, const uint16_t* wt, const
 
 int xdna_conv3x3_px_pick(int op, int B, int cin, int cout, int H, int W, int layout) {
   if (B < 1 || cin < 1 || cout < 1 || H < 1 || W < 1 || (layout != kLayoutRef && layout != kLayoutTight)) return 0;
-  if (op < 3 && g_rows_variant.load() != 0) return 0;
-  if (op >= 3 && (g_wgrad_rows_form.load() != 0 || g_wgrad_tile.load() != 0)) return 0;
-  const int form = op == 0 || op == 3 ? kPxStride1 : op == 2 ? kPxS2Dgrad : kPxStride2;
-  if (op < 0 || op > 4 || !conv_px_fits(form, B, cin, cout, H, W, layout)) return 0;
-  if (op >= 3 && !conv_px_wgrad_fits(form, B, cin, cout, H, W, layout)) return 0;
-  if (op == 1 || op == 2 || op == 4) return 1;
+  const bool wgrad = op == 3 || op == 4;
+  if (!wgrad && g_rows_variant.load() != 0) return 0;
+  if (wgrad && (g_wgrad_rows_form.load() != 0 || g_wgrad_tile.load() != 0)) return 0;
+  const int form = op == 0 || op == 3 || op == 5 ? kPxStride1 : op == 2 ? kPxS2Dgrad : kPxStride2;
+  if (op < 0 || op > 6 || !conv_px_fits(form, B, cin, cout, H, W, layout)) return 0;
+  if (wgrad && !conv_px_wgrad_fits(form, B, cin, cout, H, W, layout)) return 0;
+  if (op == 2 || op == 4) return 1;
+  const ConvGeom geom = conv_geom(B, H, W, layout);
+  const int64_t chunks = ceil_div(cin, kKStep), wgs = ceil_div(geom.m_total, 256) * ceil_div(cout, kSCo);
+  // The stride-2 forward makes a quarter of the small-grid form's products, which is nothing to
+  // gain while those are one round of a few workgroups (32 -> 16 on 19 x 26 x 26 from NCHW in place 6.9
+  // us, packed and by pixels 11.4; 64 -> 128 on 14 x 4 x 4 6.5 / 9.0; 512 -> 64 on 6 x 16 x 16 10.8 / 14.3;
+  // but 256 -> 256 on 64 x 6 x 6 13.7 / 9.4).  Over 1100 shapes by chunks times workgroups: in place up
+  // to 100, 200 where a 64-channel tile is mostly empty or K does not split far (px 1.1-1.5 of its time;
+  // 0.5-0.9 beyond), packed up to 40 (1.05-1.15).
+  if (op == 6) return chunks * wgs > (cout <= kSCo && chunks <= 4 ? 200 : 100);
+  if (op == 1) return chunks * wgs > 40;
+  if (op == 5) {
+    // in place: up to 64 output channels the pack is most of the difference (256 -> 32 on 82 x 16 x 16 21
+    // in place / 29; 512 -> 23 on 26 x 3 x 3 8.9 / 13.3); beyond, splits of K over the pixels win from 9
+    // workgroups on (512 -> 256 on 40 x 4 x 4 23.1 / 16.8), from 70 on with fewer than 5 chunks
+    // (256ch 40 x 9 x 9 19.3 / 16.1, 256 -> 128 on 1 x 35 x 35 11.2 / 14.2)
+    return cin > 3 * kKStep && cout > kSCo && wgs >= (chunks > 4 ? 9 : 70) && wgs < 150;
+  }
   if (op == 0) {
-    // grids the window kernels leave to their small-grid form, from 256 input channels: 256ch
-    // 40 x 9 x 9 13.4 -> 12.5 us (and 16.1 with the pack, where the form reading NCHW in place
-    // takes 19.3), 512 -> 256 at 40 x 4 x 4 16.8 -> 11.4 (23.1 in place); with fewer chunks the
-    // window's reuse by its nine taps is worth more (128ch 40 x 9 x 9 7.0 against 10.1)
-    const ConvGeom g = conv_geom(B, H, W, layout);
-    return cin > 3 * kKStep && ceil_div(g.m_total, 256) * ceil_div(cout, kSCo) < 150;
+    // grids the window kernels leave to their small-grid form, from 256 input channels and 9 of its
+    // workgroups: 256ch 40 x 9 x 9 13.4 -> 12.5 us, 512 -> 256 at 40 x 4 x 4 16.8 -> 11.4; with fewer
+    // chunks the window's reuse by its nine taps is worth more (128ch 40 x 9 x 9 7.0 against 10.1)
+    return cin > 3 * kKStep && wgs > 8 && wgs < 150;
   }
   // the weight gradient, on `border` packed rows per pixel: the window kernels have the higher
   // rate once work fills the chip (1.2 against 0.87 PFLOP/s), this one wastes neither border

@@ -522,14 +522,15 @@ std::atomic<int> g_conv_nchw{[] {
 
 // Where the real-pixel kernels are the better choice (xdna_conv3x3_px_pick's ops), for a conv
 // of the H x W image sizes[2] x sizes[3].
-enum PxOp { kPxFwd = 0, kPxS2Fwd = 1, kPxS2Dx = 2, kPxDw = 3, kPxS2Dw = 4 };
+// (the last two: with the pack, against the kernel that reads NCHW in place)
+enum PxOp { kPxFwd = 0, kPxS2Fwd = 1, kPxS2Dx = 2, kPxDw = 3, kPxS2Dw = 4, kPxFwdNchw = 5, kPxS2FwdNchw = 6 };
 bool px_pick(PxOp op, at::IntArrayRef sizes, int64_t cin, int64_t cout, int layout) {
   return xdna_conv3x3_px_pick(op, int(sizes[0]), int(cin), int(cout), int(sizes[2]), int(sizes[3]), layout) == 1;
 }
 
 bool nchw_route(const at::Tensor& src, int64_t cout, bool s1) {
   if (!g_conv_nchw.load() || (s1 && g_bfp16_emul.load())) return false;
-  if (px_pick(s1 ? kPxFwd : kPxS2Fwd, src.sizes(), src.size(1), cout, g_conv_layout.load())) return false;
+  if (px_pick(s1 ? kPxFwdNchw : kPxS2FwdNchw, src.sizes(), src.size(1), cout, g_conv_layout.load())) return false;
   return xdna_conv3x3_nchw_small_eligible(int(src.size(0)), int(src.size(1)), int(cout), int(src.size(2)),
                                           int(src.size(3))) == 1;
 }

@@ -58,6 +58,26 @@ def test_few_channel_convs_take_the_faster_form(shape, here, other):
     assert (got > 0) == (here < other)
 
 
+# op (0 / 1 stride-1 / stride-2 forward against the packed-rows kernels, 5 / 6 with the pack against the one that
+# reads NCHW in place), B, Cin, Cout, H, W: us of the real-pixel kernel, us of the other
+PX = [
+    ((6, 19, 32, 16, 26, 26), 11.4, 6.9), ((6, 14, 64, 128, 4, 4), 9.0, 6.5), ((6, 1, 16, 512, 28, 28), 10.8, 6.7),
+    ((6, 6, 512, 64, 16, 16), 14.3, 10.8), ((6, 572, 128, 16, 3, 3), 16.2, 9.2), ((6, 68, 128, 64, 2, 2), 12.6, 10.7),
+    ((1, 1, 9, 128, 37, 5), 10.2, 8.6), ((1, 3, 7, 256, 24, 24), 11.0, 9.5),
+    ((6, 40, 64, 128, 18, 18), None, None), ((1, 128, 64, 128, 64, 64), 57, 72), ((1, 40, 32, 64, 36, 36), None, None),
+    ((5, 6, 512, 5, 6, 6), 13.0, 8.5), ((5, 82, 256, 32, 16, 16), 28.7, 20.9), ((5, 1909, 256, 64, 2, 2), 30.6, 20.7),
+    ((5, 1, 256, 128, 35, 35), 14.2, 11.2), ((5, 4, 512, 64, 10, 7), 13.1, 8.9), ((0, 26, 512, 23, 3, 3), 9.1, 8.1),
+    ((5, 40, 256, 256, 9, 9), 16.1, 19.3), ((5, 40, 512, 256, 4, 4), 16.8, 23.1), ((0, 40, 256, 256, 9, 9), 12.5, 13.4),
+    ((0, 40, 512, 256, 4, 4), 11.4, 16.8), ((0, 40, 128, 128, 9, 9), 10.1, 7.0),
+]
+
+
+@pytest.mark.parametrize("shape,here,other", PX, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "")
+def test_conv3x3_forwards_take_the_faster_form(shape, here, other):
+    want = 1 if here is None or here < other else 0
+    assert hip_abi.load().xdna_conv3x3_px_pick(*shape, 1) == want
+
+
 def test_grids_past_the_launch_limit_stay_off_the_few_channel_kernels():
     """A workgroup per image of 256 threads: 2^24 of them are more threads than a launch takes."""
     lib = hip_abi.load()

@@ -1,11 +1,11 @@
-"""3x3 / stride-2 / pad-1 convs on the xdna device, run through the stride-1 conv kernels
-(forward = the even outputs of the stride-1 conv, stored straight into the strided
-output; gradients = the stride-1 gradients of the gradient spread onto the stride-1 grid
-with zeros, packed in one pass), against the float64 oracle of the strided conv, to the
-conv bar: 2 bf16 ulp (floor at ulp(max|ref| * 2^-8)) and relative L2 <= 1e-2.  Shapes:
-the style encoder's two strided layers, ResNet's downsampling conv, odd sizes (ceil(H/2)
-outputs) and non-square images.  The two entry points of that path are checked bit for
-bit against the sampling kernels they replace."""
+"""3x3 / stride-2 / pad-1 convs on the xdna device, against the float64 oracle of the strided conv,
+to the conv bar: 2 bf16 ulp (floor at ulp(max|ref| * 2^-8)) and relative L2 <= 1e-2.  Every route of
+such a layer: the choice's own (real-pixel kernels, for small forwards the stride-1 kernels storing
+only the even outputs), the stride-1 form throughout (even outputs; gradients of the gradient
+spread onto the stride-1 grid with zeros, packed in one pass), and the real-pixel forward
+with the spread gradients.  Shapes: the style encoder's two strided layers, ResNet's
+downsampling conv, odd sizes (ceil(H/2) outputs), non-square images.  The two entry points of the
+stride-1 form are checked bit for bit against the sampling kernels they replace."""
 import numpy as np
 import pytest
 import torch
@@ -24,11 +24,27 @@ def bits(t):
     return t.detach().cpu().contiguous().view(torch.int16).numpy().view(np.uint16)
 
 
+@pytest.fixture(params=["auto", "stride-1 form", "spread gradients"])
+def route(request):
+    """The route of a stride-2 layer: a forced rows kernel turns every real-pixel kernel but the weight
+    gradient's off, a forced weight-gradient kernel that one, and with it the input gradient's."""
+    lib = hip_abi.load()
+    if request.param == "stride-1 form":
+        assert lib.xdna_conv3x3_set_rows_variant(9) == 0
+    elif request.param == "spread gradients":
+        assert lib.xdna_conv3x3_set_wgrad_rows_kernel(2) == 0
+    yield request.param
+    assert lib.xdna_conv3x3_set_rows_variant(0) == 0 and lib.xdna_conv3x3_set_wgrad_rows_kernel(0) == 0
+
+
 @pytest.mark.parametrize("shape", [(4, 32, 64, 36, 36), (4, 64, 128, 18, 18), (2, 64, 128, 16, 16),
-                                   (3, 5, 7, 13, 11), (1, 3, 64, 9, 20)])
-def test_stride2_conv_matches_oracle(shape):
+                                   (3, 5, 7, 13, 11), (1, 3, 64, 9, 20), (16, 64, 72, 29, 31)])
+def test_stride2_conv_matches_oracle(shape, route):
     B, cin, cout, H, W = shape
-    print(f"conv3x3 s2 {shape}", flush=True)
+    print(f"conv3x3 s2 {shape} {route}", flush=True)
+    picks = [hip_abi.load().xdna_conv3x3_px_pick(op, B, *((cout, cin) if op == 2 else (cin, cout)), H, W, 1) for op in (1, 2, 4)]
+    assert picks[1:] == {"auto": [1, 1], "stride-1 form": [0, 1], "spread gradients": [1, 0]}[route]
+    assert picks[0] == (1 if B == 16 and route != "stride-1 form" else 0)
     torch.manual_seed(sum(shape))
     conv = nn.Conv2d(cin, cout, 3, stride=2, padding=1).bfloat16()
     x = torch.randn(B, cin, H, W).bfloat16()
@@ -51,6 +67,24 @@ def test_stride2_conv_matches_oracle(shape):
     gw, gb = oracle.conv2d_wgrad(xb, dyb, (3, 3), (2, 2), (1, 1))
     check_bf16(bits(cd.weight.grad), gw, what=f"wgrad {shape}")
     check_bf16(bits(cd.bias.grad), gb, what=f"bias grad {shape}")
+
+
+@pytest.mark.parametrize("shape", [(4, 32, 64, 36, 36), (3, 8, 7, 13, 11), (16, 64, 72, 29, 31)])
+def test_stride2_forward_of_a_frozen_layer(shape, route):
+    """Without a pack to keep, a small forward reads NCHW in place."""
+    B, cin, cout, H, W = shape
+    print(f"conv3x3 s2 frozen {shape} {route}", flush=True)
+    torch.manual_seed(sum(shape) + 1)
+    conv = nn.Conv2d(cin, cout, 3, stride=2, padding=1).bfloat16().requires_grad_(False)
+    x = torch.randn(B, cin, H, W).bfloat16()
+    ref = oracle.conv2d_fwd(bits(x), bits(conv.weight), bits(conv.bias), (2, 2), (1, 1))
+    xdna_train.reset_mapped_cpu_stats()
+    y = conv.to(X)(x.to(X))
+    torch.xdna.synchronize()
+    st = xdna_train.mapped_cpu_stats()
+    in_place = st.get("hip_conv3x3.nchw", {}).get("calls", 0)
+    assert in_place == (1 if B < 16 and route != "stride-1 form" else 0), st
+    check_bf16(bits(y), ref, what=f"fwd {shape}")
 
 
 @pytest.mark.parametrize("H,W", [(7, 10), (16, 16), (9, 12), (36, 36), (64, 64), (5, 4)])
