@@ -86,24 +86,21 @@ struct BwdArgs {
   int H, W, Ho, Wo;
 };
 
-// Four values from p, of which n are in the tensor (the others are 0).
-struct Vals4 {
-  float v[4];
-};
-
-__device__ inline Vals4 load4(const uint16_t* p, int n) {
-  Vals4 o = {{0.0f, 0.0f, 0.0f, 0.0f}};
-  if (n >= 4) {
-    const Pix4 a = *reinterpret_cast<const Pix4*>(p);
-    o.v[0] = bf16_to_f32(uint16_t(a.lo)), o.v[1] = bf16_to_f32(uint16_t(a.lo >> 16));
-    o.v[2] = bf16_to_f32(uint16_t(a.hi)), o.v[3] = bf16_to_f32(uint16_t(a.hi >> 16));
-  } else {
-#pragma unroll
-    for (int u = 0; u < 3; ++u)
-      if (u < n) o.v[u] = bf16_to_f32(p[u]);
+// The four elements from i of a tensor of `total` in the low bits on (past the last: anything).  The
+// load is whole and unconditional, so that a kernel's loads fly together: one that ends past the
+// tensor is moved back and shifted.  Tensors of fewer than four elements are read one by one.
+__device__ inline uint64_t load4(const uint16_t* p, int64_t i, int64_t total) {
+  if (total < 4) {
+    uint64_t v = 0;
+    for (int u = 0; i + u < total; ++u) v |= uint64_t(p[i + u]) << (16 * u);
+    return v;
   }
-  return o;
+  const int64_t b = i < total - 4 ? i : total - 4;
+  const Pix4 a = *reinterpret_cast<const Pix4*>(p + b);
+  return (a.lo | (uint64_t(a.hi) << 32)) >> (16 * int(i - b));
 }
+
+__device__ inline float val4(uint64_t v, int u) { return bf16_to_f32(uint16_t(v >> (16 * u))); }
 
 __device__ inline void store4(uint16_t* p, int n, const float (&v)[4]) {
   uint16_t h[4];
@@ -118,22 +115,25 @@ __device__ inline void store4(uint16_t* p, int n, const float (&v)[4]) {
   }
 }
 
-// The mask and the terms beside the base gradient of n elements from i.
-__device__ inline void region_terms(const BwdArgs& a, float s, int64_t i, int n, float (&v)[4]) {
-  if (a.extra) {
-    const Vals4 e = load4(a.extra + i, n);
+// The mask and the terms beside the base gradient of four elements: loaded, then applied.
+struct Terms4 {
+  uint64_t extra, ta, tb, r;
+};
+
+__device__ inline Terms4 load_terms(const BwdArgs& a, int64_t i, int64_t total) {
+  Terms4 t = {0, 0, 0, 0};
+  if (a.extra) t.extra = load4(a.extra, i, total);
+  if (a.ta) t.ta = load4(a.ta, i, total), t.tb = load4(a.tb, i, total);
+  if (a.r) t.r = load4(a.r, i, total);
+  return t;
+}
+
+__device__ inline void region_terms(const BwdArgs& a, float s, const Terms4& t, float (&v)[4]) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] += e.v[u];
-  }
-  if (a.ta) {
-    const Vals4 x = load4(a.ta + i, n), y = load4(a.tb + i, n);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] += s * (x.v[u] - y.v[u]);
-  }
-  if (a.r) {
-    const Vals4 r = load4(a.r + i, n);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = r.v[u] <= 0.0f ? 0.0f : v[u];
+  for (int u = 0; u < 4; ++u) {
+    if (a.extra) v[u] += val4(t.extra, u);
+    if (a.ta) v[u] += s * (val4(t.ta, u) - val4(t.tb, u));
+    if (a.r) v[u] = val4(t.r, u) <= 0.0f ? 0.0f : v[u];
   }
 }
 
@@ -146,16 +146,42 @@ __global__ __launch_bounds__(kRegionThreads) void region_bwd_kernel(BwdArgs a) {
   const float s = a.ta ? a.scale * go_value(a.go, a.go_dtype) : 0.0f;
   for (int64_t i = (int64_t(blockIdx.x) * kRegionThreads + threadIdx.x) * 4; i < n;
        i += int64_t(gridDim.x) * kRegionThreads * 4) {
-    const int m = int(std::min<int64_t>(4, n - i));
-    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (a.g) {
-      const Vals4 g = load4(a.g + i, m);
+    const uint64_t g = a.g ? load4(a.g, i, n) : 0;
+    const Terms4 t = load_terms(a, i, n);
+    float v[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = g.v[u];
-    }
-    region_terms(a, s, i, m, v);
-    store4(a.out + i, m, v);
+    for (int u = 0; u < 4; ++u) v[u] = val4(g, u);
+    region_terms(a, s, t, v);
+    store4(a.out + i, int(std::min<int64_t>(4, n - i)), v);
   }
+}
+
+// One element per thread, through the max-pool too: small tensors, where the other forms' longer
+// code, not memory, is the time (with the pool, extra and a mask 3.1 us against 4.1 up to 100k
+// elements, level at 400k; without the pool, with extra and a tap, 2.9 against 3.2, level at 200k).
+__global__ __launch_bounds__(kRegionThreads) void region_bwd_small_kernel(BwdArgs a) {
+  const int n = int(a.planes * a.H * a.W), i = int(blockIdx.x) * kRegionThreads + int(threadIdx.x);
+  if (i >= n) return;
+  const float s = a.ta ? a.scale * go_value(a.go, a.go_dtype) : 0.0f;
+  if (a.r && bf16_to_f32(a.r[i]) <= 0.0f) {
+    a.out[i] = 0;
+    return;
+  }
+  float v = 0.0f;
+  if (a.g) {
+    v = bf16_to_f32(a.g[i]);
+  } else if (a.gp) {
+    const int row = i / a.W, x = i - row * a.W, p = row / a.H, y = row - p * a.H;
+    const int oy = y >> 1, ox = x >> 1;
+    if (oy < a.Ho && ox < a.Wo) {
+      const uint16_t* w0 = a.px + (p * a.H + 2 * oy) * a.W + 2 * ox;
+      const float w[4] = {bf16_to_f32(w0[0]), bf16_to_f32(w0[1]), bf16_to_f32(w0[a.W]), bf16_to_f32(w0[a.W + 1])};
+      if (argmax4(w) == ((y & 1) << 1) + (x & 1)) v = bf16_to_f32(a.gp[(p * a.Ho + oy) * a.Wo + ox]);
+    }
+  }
+  if (a.extra) v += bf16_to_f32(a.extra[i]);
+  if (a.ta) v += s * (bf16_to_f32(a.ta[i]) - bf16_to_f32(a.tb[i]));
+  a.out[i] = f32_to_bf16(v);
 }
 
 // Through the max-pool: a thread takes four columns of the two rows of a window row, so a
@@ -164,6 +190,7 @@ __global__ __launch_bounds__(kRegionThreads) void region_bwd_kernel(BwdArgs a) {
 template <class I>
 __global__ __launch_bounds__(kRegionThreads) void region_bwd_pool_kernel(BwdArgs a) {
   const I wq = I((a.W + 3) / 4), hq = I((a.H + 1) / 2), n = I(a.planes) * hq * wq;
+  const int64_t total = a.planes * a.H * a.W, pooled = a.planes * a.Ho * a.Wo;
   const float s = a.ta ? a.scale * go_value(a.go, a.go_dtype) : 0.0f;
   for (I i = I(blockIdx.x) * kRegionThreads + threadIdx.x; i < n; i += I(gridDim.x) * kRegionThreads) {
     const I row = i / wq;
@@ -172,27 +199,29 @@ __global__ __launch_bounds__(kRegionThreads) void region_bwd_pool_kernel(BwdArgs
     const int oy = int(row - p * hq), y = 2 * oy, m = min(4, a.W - x);
     const int64_t at = (int64_t(p) * a.H + y) * a.W + x;
     const bool two = y + 1 < a.H;
+    const int64_t below = two ? at + a.W : at;
+    const uint64_t r0 = load4(a.px, at, total), r1 = load4(a.px, below, total);
+    const Terms4 t0 = load_terms(a, at, total), t1 = load_terms(a, below, total);
+    // (the windows of the two column pairs; past the last one: anything)
+    const int64_t gi = (int64_t(p) * a.Ho + oy) * a.Wo + (x >> 1);
+    const float g[2] = {pooled ? bf16_to_f32(a.gp[gi < pooled ? gi : pooled - 1]) : 0.0f,
+                        pooled ? bf16_to_f32(a.gp[gi + 1 < pooled ? gi + 1 : pooled - 1]) : 0.0f};
     float v[2][4] = {};
-    if (two) {
-      const Vals4 r0 = load4(a.px + at, m), r1 = load4(a.px + at + a.W, m);
-      const uint16_t* gp = a.gp + (int64_t(p) * a.Ho + oy) * a.Wo + (x >> 1);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if (2 * j + 1 >= m) continue;  // no window (an odd last column)
-        const float w[4] = {r0.v[2 * j], r0.v[2 * j + 1], r1.v[2 * j], r1.v[2 * j + 1]};
-        const float g = bf16_to_f32(gp[j]);
-        const int k = argmax4(w);
-        v[0][2 * j] = k == 0 ? g : 0.0f;
-        v[0][2 * j + 1] = k == 1 ? g : 0.0f;
-        v[1][2 * j] = k == 2 ? g : 0.0f;
-        v[1][2 * j + 1] = k == 3 ? g : 0.0f;
-      }
+    for (int j = 0; j < 2; ++j) {
+      if (!two || 2 * j + 1 >= m) continue;  // no window (an odd last row or column)
+      const float w[4] = {val4(r0, 2 * j), val4(r0, 2 * j + 1), val4(r1, 2 * j), val4(r1, 2 * j + 1)};
+      const int k = argmax4(w);
+      v[0][2 * j] = k == 0 ? g[j] : 0.0f;
+      v[0][2 * j + 1] = k == 1 ? g[j] : 0.0f;
+      v[1][2 * j] = k == 2 ? g[j] : 0.0f;
+      v[1][2 * j + 1] = k == 3 ? g[j] : 0.0f;
     }
-    region_terms(a, s, at, m, v[0]);
+    region_terms(a, s, t0, v[0]);
     store4(a.out + at, m, v[0]);
     if (two) {
-      region_terms(a, s, at + a.W, m, v[1]);
-      store4(a.out + at + a.W, m, v[1]);
+      region_terms(a, s, t1, v[1]);
+      store4(a.out + below, m, v[1]);
     }
   }
 }
@@ -231,31 +260,59 @@ __global__ __launch_bounds__(kRegionThreads) void sqdiff_kernel(const uint16_t* 
 
 // The same of (G / chw - t)^2: G the bf16 Gram matrices [batch][cc], t fp32 targets with batch
 // stride t_bstride, 0 for one target broadcast over the batch.  A thread sums runs of eight (at
-// 8 (b * 256 + tid) + k * gridDim.x * 2048) in order; a run lies in one matrix where cc % 8 == 0,
-// so its index is divided once, in 32 bits where it fits (a 64-bit division per element held
-// 40 matrices of 512 x 512 to 14.2 us; now 8.0, the bytes' time is 4).
+// 8 (b * 256 + tid) + k * gridDim.x * 2048) in order, each divided once, in 32 bits where it fits (a
+// 64-bit division per element held 40 matrices of 512 x 512 to 14.2 us; now 8.0, the bytes' time is
+// 4; 30 of 471 x 471 10.7).  A run that crosses into the next matrix, or ends the last, is read
+// element by element, all loads in flight.
+// kSmall: no more elements than threads, one each (3.3 us; the runs' code alone 0.2-0.9 more).
+template <bool kSmall>
 __global__ __launch_bounds__(kRegionThreads) void gram_sqdiff_kernel(const uint16_t* __restrict__ G,
                                                                      const float* __restrict__ t, int64_t t_bstride,
                                                                      int64_t cc, float chw, int64_t n, float scale,
                                                                      float* __restrict__ part) {
   float s = 0.0f;
+  if constexpr (kSmall) {
+    const uint32_t i = blockIdx.x * kRegionThreads + threadIdx.x;
+    if (i < n) {
+      const uint32_t bi = i / uint32_t(cc);
+      const float d = bf16_to_f32(G[i]) / chw - t[bi * t_bstride + (i - bi * cc)];
+      s = d * d;
+    }
+    block_part(s, scale, part);
+    return;
+  }
   for (int64_t i = (int64_t(blockIdx.x) * kRegionThreads + threadIdx.x) * 8; i < n;
        i += int64_t(gridDim.x) * kRegionThreads * 8) {
-    if (i + 8 <= n && cc % 8 == 0) {
+    const int64_t bi = (i | cc) >> 32 ? i / cc : uint32_t(i) / uint32_t(cc);
+    const float* tp = t + bi * t_bstride;
+    int64_t r = i - bi * cc;
+    float g[8], w[8];
+    if (r + 8 <= cc) {  // (then i + 8 <= n)
       const Pix8 x = *reinterpret_cast<const Pix8*>(G + i);
-      const int64_t bi = (i | cc) >> 32 ? i / cc : uint32_t(i) / uint32_t(cc);
-      const float* tp = t + bi * t_bstride + (i - bi * cc);
-      const F32x4 lo = *reinterpret_cast<const F32x4*>(tp), hi = *reinterpret_cast<const F32x4*>(tp + 4);
+      const F32x4 lo = *reinterpret_cast<const F32x4*>(tp + r), hi = *reinterpret_cast<const F32x4*>(tp + r + 4);
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const float d = bf16_to_f32(uint16_t(x.v[u >> 1] >> (16 * (u & 1)))) / chw - (u < 4 ? lo.v[u & 3] : hi.v[u & 3]);
+        g[u] = bf16_to_f32(uint16_t(x.v[u >> 1] >> (16 * (u & 1))));
+        w[u] = u < 4 ? lo.v[u & 3] : hi.v[u & 3];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float d = g[u] / chw - w[u];
         s = fmaf(d, d, s);
       }
     } else {
-      for (int64_t e = i; e < i + 8 && e < n; ++e) {
-        const int64_t bi = e / cc;
-        const float d = bf16_to_f32(G[e]) / chw - t[bi * t_bstride + (e - bi * cc)];
-        s = fmaf(d, d, s);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const bool in = i + u < n;  // (past the end: the run's first element again)
+        const float* tu = in ? tp + r : t;
+        g[u] = bf16_to_f32(G[in ? i + u : i]);
+        w[u] = *tu;
+        if (++r == cc) r = 0, tp += t_bstride;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float d = g[u] / chw - w[u];
+        if (i + u < n) s = fmaf(d, d, s);
       }
     }
   }
@@ -314,22 +371,24 @@ __global__ __launch_bounds__(kRegionThreads) void gram_grad_kernel(const uint16_
   __shared__ float tile[2][kGT][kGT + 1];
   const int y = threadIdx.x / 8, x = 4 * (threadIdx.x % 8);
   float d[2][4];
+  const bool whole = (tj + 1) * kGT <= C;  // (ti <= tj) else elements, clamped: what is past the matrix is not stored
 #pragma unroll
   for (int h = 0; h < 2; ++h) {  // the tile, its mirror
     const int r = (h ? tj : ti) * kGT + y, col = (h ? ti : tj) * kGT + x;
-    const int64_t e = int64_t(r) * C + col;
-    const int m = r < C ? C - col : 0;
-    const Vals4 g = load4(Gb + e, m);
-    F32x4 w = {{0.0f, 0.0f, 0.0f, 0.0f}};
-    if (m >= 4) {
-      w = *reinterpret_cast<const F32x4*>(tb + e);
-    } else {
+    float g[4], w[4];
+    if (whole) {
+      const int64_t e = int64_t(r) * C + col;
+      const Pix4 q = *reinterpret_cast<const Pix4*>(Gb + e);
+      const F32x4 f = *reinterpret_cast<const F32x4*>(tb + e);
 #pragma unroll
-      for (int u = 0; u < 3; ++u)
-        if (u < m) w.v[u] = tb[e + u];
+      for (int u = 0; u < 4; ++u) g[u] = bf16_to_f32(uint16_t((u < 2 ? q.lo : q.hi) >> (16 * (u & 1)))), w[u] = f.v[u];
+    } else {
+      const int64_t row = int64_t(min(r, C - 1)) * C;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) g[u] = bf16_to_f32(Gb[row + min(col + u, C - 1)]), w[u] = tb[row + min(col + u, C - 1)];
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) tile[h][y][x + u] = d[h][u] = g.v[u] / chw - w.v[u];
+    for (int u = 0; u < 4; ++u) tile[h][y][x + u] = d[h][u] = g[u] / chw - w[u];
   }
   __syncthreads();
 #pragma unroll
@@ -385,7 +444,9 @@ int xdna_region_backward_bf16(const uint16_t* r, const uint16_t* g, const uint16
   }
   if (!admit_launch("xdna_region_backward_bf16")) return -1;
   BwdArgs a{r, g, gp, px, extra, ta, tb, go, go_dtype, scale, out, planes, H, W, H / 2, W / 2};
-  if (!g && gp) {
+  if (n <= (!g && gp ? 400000 : 200000)) {
+    region_bwd_small_kernel<<<unsigned(ceil_div(n, kRegionThreads)), kRegionThreads, 0, as_stream(stream)>>>(a);
+  } else if (!g && gp) {
     const int64_t items = planes * ceil_div(H, 2) * ceil_div(W, 4);
     if (items < (int64_t(1) << 31))
       region_bwd_pool_kernel<uint32_t><<<grid_for(items), kRegionThreads, 0, as_stream(stream)>>>(a);
@@ -417,8 +478,11 @@ int xdna_region_gram_sqdiff_bf16(const uint16_t* G, const float* t, int64_t t_bs
     return -1;
   }
   if (!admit_launch("xdna_region_gram_sqdiff_bf16")) return -1;
-  gram_sqdiff_kernel<<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(G, t, t_bstride, cc, chw, batch * cc,
-                                                                          scale, part);
+  const int64_t n = batch * cc;
+  if (n <= int64_t(kLossParts) * kRegionThreads)
+    gram_sqdiff_kernel<true><<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(G, t, t_bstride, cc, chw, n, scale, part);
+  else
+    gram_sqdiff_kernel<false><<<kLossParts, kRegionThreads, 0, as_stream(stream)>>>(G, t, t_bstride, cc, chw, n, scale, part);
   return check_launch("xdna_region_gram_sqdiff_bf16");
 }
 

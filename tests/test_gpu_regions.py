@@ -352,7 +352,10 @@ def test_region_step_captured_and_replayed():
 # remainder, operands 2 bytes off a 4-byte address, planes of odd sizes (pixels without a window),
 # one row or column, Gram matrices of an odd, an even and one number of 32 x 32 tiles.
 @pytest.mark.parametrize("shape,off", [((2, 3, 7, 9), 1), ((1, 2, 5, 6), 0), ((3, 1, 2, 3), 1), ((1, 4, 1, 8), 0),
-                                       ((2, 2, 9, 1), 0), ((1, 1, 4, 11), 1), ((1, 1, 64, 37), 0)])
+                                       ((2, 2, 9, 1), 0), ((1, 1, 4, 11), 1), ((1, 1, 64, 37), 0),
+                                       # past the element-by-element form's sizes
+                                       ((1, 300, 37, 41), 1), ((7, 70, 33, 26), 0), ((900, 64, 3, 3), 1),
+                                       ((1000, 64, 9, 1), 0), ((100, 2500, 1, 2), 1), ((50, 70, 8, 16), 0)])
 def test_backward_pass_edges(shape, off):
     g = torch.Generator().manual_seed(31 + sum(shape))
 
@@ -381,7 +384,9 @@ def test_backward_pass_edges(shape, off):
 
 
 @pytest.mark.parametrize("B,n,per_batch,off", [(3, 1, False, 0), (2, 31, True, 1), (1, 32, False, 0), (2, 66, True, 0),
-                                               (1, 97, True, 1), (2, 128, True, 0)])
+                                               (1, 97, True, 1), (2, 128, True, 0),
+                                               # more elements than threads: runs that cross matrices, and not
+                                               (60000, 3, True, 1), (600, 31, True, 0), (130, 66, False, 1), (9, 256, True, 0)])
 def test_gram_term_edges(B, n, per_batch, off):
     g = torch.Generator().manual_seed(n)
 
