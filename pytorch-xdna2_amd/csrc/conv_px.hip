@@ -632,9 +632,14 @@ int conv_px(int form, const uint16_t* xp, const uint16_t* wt, const uint16_t* bi
 
 bool conv_px_wgrad_fits(int form, int B, int Cin, int Cout, int H, int W, int layout) {
   const int Ho = form == kPxStride2 ? (H + 1) / 2 : H, Wo = form == kPxStride2 ? (W + 1) / 2 : W;
-  // (dY's packed rows are the operand of a stride-1 conv of it; a split's table holds kPwMaxKt
-  // k-tiles, so more pixels than kPwMaxSplits of them have no plan)
-  return conv_px_fits(form, B, Cin, Cout, H, W, layout) && conv_px_fits(kPxStride1, B, Cout, Cin, H, W, layout) &&
+  const ConvGeom g = conv_geom(B, H, W, layout), d = conv_geom(B, Ho, Wo, layout);
+  const int64_t ci = ceil_div(Cin, 64), co = ceil_div(Cout, 64);
+  // What it addresses: the packed rows of x and of dY, both ending before the out-of-range row
+  // offset, and partials the size of the weight.  A split's table holds kPwMaxKt k-tiles, so more
+  // pixels than kPwMaxSplits of them have no plan.
+  return int64_t(g.groups) * ci * kGroupRows * kKStep * 2 < kPwOob - 4096 &&
+         int64_t(d.groups) * co * kGroupRows * kKStep * 2 < kPwOob - 4096 && g.m_total < (int64_t(1) << 31) &&
+         ci * 64 * co * 64 * 9 * 2 < (int64_t(1) << 31) &&
          ceil_div(int64_t(B) * Ho * Wo, kPwK) <= int64_t(kPwMaxSplits) * kPwMaxKt;
 }
 

@@ -84,3 +84,13 @@ def test_grids_past_the_launch_limit_stay_off_the_few_channel_kernels():
     pick = lambda op, *a: lib.xdna_conv2d_few_pick(op, *a, 3, 3, 1, 1, 1)  # noqa: E731
     assert pick(0, 1 << 24, 8, 3, 1, 4) == 0 and pick(0, 1 << 24, 3, 8, 1, 4) == 0 and pick(1, 1 << 24, 3, 8, 1, 4) == 0
     assert lib.xdna_conv1x1_pick(0, 1 << 24, 8, 8, 1, 4, 1) == 0
+
+
+def test_stride2_layers_within_the_offset_limits_take_the_real_pixel_kernels():
+    """The weight gradient's limits are those of x's and of the half-resolution dY's packed rows; past
+    them (2 GB) the layer takes the stride-1 form."""
+    pick = hip_abi.load().xdna_conv3x3_px_pick
+    assert pick(4, 128, 128, 512, 128, 128, 1) == 1 and pick(2, 128, 512, 128, 128, 128, 1) == 1
+    assert pick(4, 128, 1024, 64, 128, 128, 1) == 0  # x's rows 4.4 GB
+    assert pick(4, 500, 64, 512, 128, 128, 1) == 0   # dY's 2.3 GB
+    assert pick(3, 500, 64, 64, 128, 128, 1) == 0    # pixels: more than a plan holds

@@ -122,6 +122,42 @@ def test_pick(hip):
     assert hip.xdna_conv3x3_set_rows_variant(0) == 0
 
 
+def test_stride2_weight_gradient_near_the_offset_limit(hip):
+    """A layer whose output gradient packs to 0.6 GB as it is and to 2.4 GB spread onto the stride-1 grid: the
+    real-pixel kernels take it, and their offsets hold (first and last channels against float64)."""
+    B, cin, cout, H, W = 128, 128, 512, 128, 128
+    assert [hip.xdna_conv3x3_px_pick(op, B, *((cout, cin) if op == 2 else (cin, cout)), H, W, 1) for op in (1, 2, 4)] == [1] * 3
+    print("conv px wgrad 128 -> 512 on 128 x 128 x 128", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(B, cin, H, W, generator=g, device="cuda").bfloat16()
+    dy = torch.randn(B, cout, H // 2, W // 2, generator=g, device="cuda").bfloat16()
+
+    def pack(t):
+        b, c, h, w = t.shape
+        buf = torch.empty(hip.xdna_conv3x3_layout_packed_bytes(b, c, h, w, 1) // 2, dtype=torch.int16, device="cuda")
+        assert hip.xdna_conv3x3_layout_pack_bf16(t.data_ptr(), buf.data_ptr(), b, c, h, w, 1, stream()) == 0
+        return buf
+
+    xp, dp = pack(x), pack(dy)
+    n = hip.xdna_conv3x3_px_wgrad_workspace_bytes(1, B, cin, cout, H, W)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    gw = torch.empty(cout, cin, 3, 3, dtype=torch.bfloat16, device="cuda")
+    assert hip.xdna_conv3x3_px_wgrad_bf16(1, xp.data_ptr(), dp.data_ptr(), gw.data_ptr(), None, B, cin, cout, H, W, 1,
+                                          ws.data_ptr(), n, stream()) == 0
+    some = [0, 1, 255, 256, 510, 511]
+    ref = torch.zeros(len(some), cin, 3, 3, dtype=torch.float64, device="cuda")
+    for b in range(0, B, 16):
+        xd = torch.nn.functional.pad(x[b:b + 16].double(), [1] * 4)
+        d = dy[b:b + 16, some].double().flatten(2)
+        for i in range(3):
+            for j in range(3):
+                t = xd[:, :, i:i + H:2, j:j + W:2].flatten(2).transpose(1, 2).contiguous()
+                ref[:, :, i, j] += torch.matmul(d, t).sum(0)
+    got = gw[some].double()
+    # one bf16 rounding beside fp32 sums of 524288 products
+    assert float((got - ref).norm() / ref.norm()) < 4e-3
+
+
 @pytest.mark.parametrize("need_dx", [True, False])
 @pytest.mark.parametrize("trainable", [True, False])
 def test_aten_stride2(trainable, need_dx):
