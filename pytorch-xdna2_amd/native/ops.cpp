@@ -528,6 +528,12 @@ bool px_pick(PxOp op, at::IntArrayRef sizes, int64_t cin, int64_t cout, int layo
   return xdna_conv3x3_px_pick(op, int(sizes[0]), int(cin), int(cout), int(sizes[2]), int(sizes[3]), layout) == 1;
 }
 
+// Products of a 3x3 conv of that many output pixels, as the kernel that takes it runs them: a
+// stride-2 conv's own on the real-pixel kernels, those of the input's pixels in the stride-1 form.
+double conv3x3_flops(int64_t B, int64_t H, int64_t W, int64_t cin, int64_t cout) {
+  return 2.0 * double(B) * double(H) * double(W) * double(cin) * double(cout) * 9.0;
+}
+
 bool nchw_route(const at::Tensor& src, int64_t cout, bool s1) {
   if (!g_conv_nchw.load() || (s1 && g_bfp16_emul.load())) return false;
   if (px_pick(s1 ? kPxFwdNchw : kPxS2FwdNchw, src.sizes(), src.size(1), cout, g_conv_layout.load())) return false;
@@ -546,7 +552,7 @@ at::Tensor hip_conv_nchw(const at::Tensor& src_in, const at::Tensor& w, const at
                          : empty_xdna({B, cout, H, W}, at::kBFloat16);
   at::Tensor bc;
   if (bias) bc = bias->contiguous();
-  const double flops = 2.0 * double(B) * double(H) * double(W) * double(cin) * double(cout) * 9.0;
+  const double flops = conv3x3_flops(B, H, W, cin, cout);
   KernelTimer kt(s2out ? "conv3x3_rows.s2" : dgrad ? "conv3x3_rows.dgrad" : "conv3x3_rows.fwd", flops);
   count_call("hip_conv3x3.nchw", 0);
   check_abi(xdna_conv3x3_nchw_act_bf16(static_cast<const uint16_t*>(src.const_data_ptr()),
@@ -568,7 +574,7 @@ at::Tensor hip_conv_packed(const at::Tensor& packed, int layout, at::IntArrayRef
                          : empty_xdna({B, cout, H, W}, at::kBFloat16);
   at::Tensor bc;
   if (bias) bc = bias->contiguous();
-  const double flops = 2.0 * double(B) * double(H) * double(W) * double(cin) * double(cout) * 9.0;
+  const double flops = conv3x3_flops(B, H, W, cin, cout);
   const auto px = [&](int form) {
     check_abi(xdna_conv3x3_px_bf16(form, static_cast<const uint16_t*>(packed.const_data_ptr()),
                                    static_cast<const uint16_t*>(wt.const_data_ptr()),
@@ -578,8 +584,9 @@ at::Tensor hip_conv_packed(const at::Tensor& packed, int layout, at::IntArrayRef
               "conv pixels");
   };
   if (s2out) {
-    KernelTimer kt("conv3x3_rows.s2", flops);
-    if (px_pick(kPxS2Fwd, src, cin, cout, layout)) {
+    const bool by_pixels = px_pick(kPxS2Fwd, src, cin, cout, layout);
+    KernelTimer kt("conv3x3_rows.s2", by_pixels ? conv3x3_flops(B, (H + 1) / 2, (W + 1) / 2, cin, cout) : flops);
+    if (by_pixels) {
       px(kPxS2Fwd);
       return out;
     }
@@ -618,7 +625,8 @@ at::Tensor hip_conv_packed(const at::Tensor& packed, int layout, at::IntArrayRef
 at::Tensor hip_conv_s2_dx(const at::Tensor& dpacked, int layout, at::IntArrayRef sizes, const at::Tensor& w) {
   at::Tensor wt = conv_weight_form(w, true);
   at::Tensor dx = empty_xdna(sizes, at::kBFloat16);
-  KernelTimer kt("conv3x3_rows.dgrad", 2.0 * double(dx.numel()) * double(w.size(0)) * 9.0 / 4.0);
+  KernelTimer kt("conv3x3_rows.dgrad",
+                 conv3x3_flops(sizes[0], (sizes[2] + 1) / 2, (sizes[3] + 1) / 2, w.size(0), w.size(1)));
   check_abi(xdna_conv3x3_px_bf16(kPxS2Dx, static_cast<const uint16_t*>(dpacked.const_data_ptr()),
                                  static_cast<const uint16_t*>(wt.const_data_ptr()), nullptr,
                                  static_cast<uint16_t*>(dx.data_ptr()), int(sizes[0]), int(w.size(0)), int(w.size(1)),
@@ -1193,7 +1201,8 @@ void wgrad_rows_launch(const WgradRowsJob& j, const at::Tensor& dpacked, at::Ten
 void hip_wgrad_rows(const at::Tensor& input, const at::Tensor& dpacked, int layout, int64_t Cout, at::Tensor& gw,
                     at::Tensor* gb, int stride, bool px2) {
   const WgradRowsJob j = wgrad_rows_prepare(input, layout, Cout, gw, gb, stride, px2);
-  KernelTimer kt("conv3x3_wgrad", 2.0 * double(j.B) * double(j.H) * double(j.W) * double(j.Cin) * double(Cout) * 9.0);
+  const int64_t per = j.px == 1 ? 2 : 1;  // (input pixels per output pixel, each way)
+  KernelTimer kt("conv3x3_wgrad", conv3x3_flops(j.B, (j.H + per - 1) / per, (j.W + per - 1) / per, j.Cin, Cout));
   wgrad_rows_launch(j, dpacked, gw, gb, current_stream());
 }
 

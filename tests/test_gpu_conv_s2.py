@@ -69,6 +69,30 @@ def test_stride2_conv_matches_oracle(shape, route):
     check_bf16(bits(cd.bias.grad), gb, what=f"bias grad {shape}")
 
 
+def test_kernel_timing_counts_the_products_that_run(route):
+    """One scale for a layer's three directions: a stride-2 conv's own products on the real-pixel
+    kernels, those of the input's pixels where the stride-1 form runs."""
+    from xdna_train import device
+
+    C = device.native()
+    B, cin, cout, H, W = 16, 64, 72, 29, 31
+    print(f"conv3x3 s2 timing {route}", flush=True)
+    conv = nn.Conv2d(cin, cout, 3, stride=2, padding=1).bfloat16().to(X)
+    x = torch.randn(B, cin, H, W).bfloat16().to(X).requires_grad_()
+    C.kernel_timing(True)
+    try:
+        y = conv(x)
+        y.backward(torch.randn(y.shape).bfloat16().to(X))
+        torch.xdna.synchronize()
+        rep = dict(C.kernel_timing_report())
+    finally:
+        C.kernel_timing(False)
+    own, spread = (2.0 * B * h * w * cin * cout * 9 for h, w in ((15, 16), (H, W)))
+    want = {"conv3x3_rows.s2": spread if route == "stride-1 form" else own,
+            "conv3x3_rows.dgrad": own if route == "auto" else spread, "conv3x3_wgrad": own if route == "auto" else spread}
+    assert {k: rep[k]["work"] for k in want} == want, rep
+
+
 @pytest.mark.parametrize("shape", [(4, 32, 64, 36, 36), (3, 8, 7, 13, 11), (16, 64, 72, 29, 31)])
 def test_stride2_forward_of_a_frozen_layer(shape, route):
     """Without a pack to keep, a small forward reads NCHW in place."""
