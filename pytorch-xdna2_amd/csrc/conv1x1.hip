@@ -44,8 +44,8 @@ struct C1Args {
 
 // 8 strided pixels from (oy, ox), the p-th, of a full plane (stride 2), zeros past the plane:
 // 16 full-plane pixels per row that the 8 touch, read where that row's pixels fall on their
-// places.  `end`: pixels from the plane's start to the end of the tensor; a row that such a
-// read could leave it from, and planes under 8 columns, are read pixel by pixel.
+// places.  `end`: pixels from the plane's start to the end of the tensor; a row whose 16 pixels
+// would start before the plane or end past the tensor is read pixel by pixel.
 __device__ inline u32x4_t c1_load8_s2(const uint16_t* plane, int64_t end, int p, int oy, int ox, int P, int Wo, int W) {
   u32x4_t r = {0, 0, 0, 0};
   for (int u0 = 0; u0 < 8 && p + u0 < P;) {
@@ -437,7 +437,9 @@ C1WgPlan c1_wgrad_plan(int B, int Cin, int Cout, int P) {
 // splits cut the chain (512 -> 64 stride 2 on 39 x 7 x 10: 53 in place, 12 as a product; input
 // gradient of 85 -> 2048 on 12 x 2 x 2: 101 / 13.5), and many workgroups, or planes whose
 // pixels fill no GEMM tile, belong here (64 -> 128 stride 2 on 128 x 64 x 64 19 / 37; input gradient
-// of 1024 -> 1483 on 190 x 4 x 2 81 / 275).  For less than two workgroups per CU; the choice asks for 12 % in favour of these kernels.
+// of 1024 -> 1483 on 190 x 4 x 2 81 / 275).
+// Used below two workgroups per CU and for strided planes of short rows; the choice asks for 12 %
+// in favour of these kernels.
 double c1_mb(int64_t elements) { return 2e-6 * double(elements); }
 
 // rows beyond the first that 8 consecutive pixels of the strided plane touch

@@ -1057,13 +1057,15 @@ int xdna_conv2d_few_pick(int op, int B, int Cin, int Cout, int H, int W, int KH,
   const int v = g_conv2d_variant.load();
   if (v == 1) return 0;
   if (op < 3) return conv_few_pick(op, B, Cin, Cout, H, W, KH, KW, ph, pw, bias != 0, v == 2);
-  // Against the pack and the rows conv: up to 8 output channels leave the chunks empty, and planes
-  // past 256 columns go in strips.  A chunk of 32 channels is a round of this kernel's chain, so from
-  // 64 channels on only where the pixels hide it: us, this one / those, 3 <- 163 on 1 x 23 x 30 17.5 / 11, 1 <- 416 on
-  // 74 x 8 x 8 38 / 21, but 1 <- 289 on 92 x 34 x 18 24 / 57, 3 <- 233 on 64 x 40 x 40 0.55 of the time.  Nor for
-  // batches of planes of up to 64 pixels, one workgroup each (3 <- 57 on 733 x 4 x 4 13.6 -> 19.6).
+  // Against the pack and the rows conv: fewer than 8 output channels leave the chunks empty, and
+  // planes past 256 columns go in strips.  A chunk of 32 channels is a round of this kernel's
+  // chain, so from 64 channels on only where the pixels hide it: us, this one / those, 3 <- 163 on
+  // 1 x 23 x 30 17.5 / 11, 1 <- 416 on 74 x 8 x 8 38 / 21, but 1 <- 289 on 92 x 34 x 18 24 / 57,
+  // 3 <- 233 on 64 x 40 x 40 0.55 of the time.  Nor for batches of planes of up to 64 pixels, one
+  // workgroup each (3 <- 57 on 733 x 4 x 4 19.6 / 13.6).
   const int64_t px = int64_t(H) * W;
-  if (KH != 3 || KW != 3 || ph != 1 || pw != 1 || Cout < 8 || W > 256 || conv_few_pick(1, B, Cin, Cout, H, W, 3, 3, 1, 1, false, v == 2) != 1)
+  if (KH != 3 || KW != 3 || ph != 1 || pw != 1 || Cout < 8 || W > 256 ||
+      conv_few_pick(1, B, Cin, Cout, H, W, 3, 3, 1, 1, false, v == 2) != 1)
     return 0;
   if (v == 2 || Cout <= 32) return 1;
   return !(px <= 64 && B > 512) && (Cout <= 64 || B * px >= 75 * int64_t(Cout));

@@ -66,10 +66,12 @@ bool conv_eligible(const at::Tensor& x, const at::Tensor& w, c10::SymIntArrayRef
 
 // 3x3 / stride-2 / pad-1 convs (the style encoder, ResNet's downsampling blocks) run on the
 // real-pixel kernels (xdna_conv3x3_px_*) on the stride-1 path's packed rows and prepared
-// weights.  Operands past those kernels' 32-bit offsets, and runs that force a stride-1
-// kernel, take the stride-1 form: the conv at every other row and column, and the gradients
-// of the output gradient spread onto the stride-1 grid with zeros (4x the MACs).  The reference
-// runs them on its CPU through the fallback (torch_xdna_device.cpp:4524-4606, 4608-4885).
+// weights.  Forwards too small for those kernels (nchw_route, xdna_conv3x3_px_pick),
+// operands past their 32-bit offsets, and runs that force a stride-1 kernel, take the
+// stride-1 form: the conv at every other row and column, and the gradients of the output
+// gradient spread onto the stride-1 grid with zeros (4x the MACs).  The
+// reference runs them on its CPU through the fallback (torch_xdna_device.cpp:4524-4606,
+// 4608-4885).
 // XDNA_CONV_S2=0 sends 3x3 / stride-2 convs to the general kernels instead (their real
 // MACs on the gather GEMM), for measurements.
 const bool g_conv_s2 = [] {
@@ -871,7 +873,7 @@ bool gconv_auto(int cout, int sh, int sw) { return cout >= 32 && sh == 1 && sw =
 // gradient take the general kernels (measured on MI355X: ResNet-18's stem B128 3->64 at
 // 64x64 forward 80.6 -> 30.3 us, weight gradient 209 -> 76 us; VGG's first layer B40 at
 // 36x36 forward 19.2 -> 7.2 us).  So does their input gradient where the few-channel form
-// fits (few_input_dx): VGG's first layer 13.3 (pack and rows conv) -> 9.8 us.
+// is the faster one (few_input_dx): VGG's first layer 13.3 (pack and rows conv) -> 9.8 us.
 bool few_input_3x3(const at::Tensor& x, const at::Tensor& w) {
   const int m = g_gconv_mode.load();
   return x.size(1) <= 4 && (m == 2 || (m == 1 && gconv_auto(int(w.size(0)), 1, 1)));
@@ -1266,9 +1268,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> convolution_backward_overrideable
                      grad_output.size(1) == weight.size(0) && grad_output.size(0) == input.size(0);
   bool hip = conv_eligible(input, weight, stride, padding, dilation, transposed, output_padding, groups) &&
              go_ok && grad_output.size(2) == input.size(2) && grad_output.size(3) == input.size(3);
-  // stride 2 beside the real-pixel kernels: the stride-1 gradients of the gradient spread onto the stride-1 grid (its
-  // packed rows made in one pass; the spread tensor itself only for the channel-major
-  // weight gradient)
+  // stride 2 (px2 below: from the gradient as it is); past the real-pixel kernels the stride-1
+  // gradients of the gradient spread onto the stride-1 grid (its packed rows made in one pass;
+  // the spread tensor itself only for the channel-major weight gradient)
   at::Tensor go = grad_output;
   bool strided = false;
   std::vector<int64_t> go_sizes = grad_output.sizes().vec();

@@ -7,9 +7,10 @@ ResNet's 7x7 stride-2 stem and 1x1 stride-2 downsampling, non-square kernels and
 strides, odd sizes, channel counts that leave partial 32 / 64 / 128-row tiles, and a
 pixel count beyond one 128-column tile row.  The weight gradient is checked for
 run-to-run bit equality (fixed-order split reduction).  Forward and input gradient run
-in both kernel forms: automatic (the direct form at stride 1 with <= 32 output and >= 16
-input channels of the direction, up to the widest padded row it stages) and the gather
-GEMM alone.
+in both kernel forms: automatic (the few-channel kernels where they are the faster ones,
+else the direct form at stride 1 with <= 32 output and >= 16 input channels of the
+direction, up to the widest padded row it stages) and the gather GEMM alone; the
+few-channel kernels wherever they apply have a test of their own.
 """
 import numpy as np
 import pytest
